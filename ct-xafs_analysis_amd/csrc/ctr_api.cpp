@@ -66,6 +66,7 @@ struct SliceSet {
     const int *d_map[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
     int nb[6] = {0, 0, 0, 0, 0, 0};
     int fp_wpb = 4, fp_rays = 64, fp_tile = 60, bp_rows = 4, na = 1;
+    bool quad = false;       // descriptors are quads (four interleaved slices each)
     // the maps in `dev` and what they were planned from (the schedule and
     // every slice's extents); own_at is null when dev holds no valid maps
     std::vector<int> map_sig;
@@ -128,6 +129,18 @@ Layout make_layout(int nx, int ny, int px)
     l.rpitch = round_up(px + 2 * l.roff, 16);
     return l;
 }
+
+// The layout of a quad: pitches in texels of QZ floats, a wider frame.
+Layout make_quad_layout(int nx, int ny, int px)
+{
+    Layout l = make_layout(nx, ny, px);
+    l.ipitch = round_up(nx + 2 * QPAD, 16);
+    l.tpitch = round_up(ny + 2 * QPAD, 16);
+    return l;
+}
+
+size_t quad_img_floats(const Layout &l) { return (size_t)QZ * (l.ny + 2 * QPAD) * l.ipitch; }
+size_t quad_imgT_floats(const Layout &l) { return (size_t)QZ * (l.nx + 2 * QPAD) * l.tpitch; }
 
 size_t pimg_floats(const Layout &l) { return (size_t)(l.ny + 2 * PAD) * l.ipitch; }
 size_t pimgT_floats(const Layout &l) { return (size_t)(l.nx + 2 * PAD) * l.tpitch; }
@@ -210,6 +223,7 @@ struct ctr_ctx {
     DevBuf w_xproj, w_stage; // sinogram formation: x-projections, sinograms before spike removal
     DevBuf w_gpad;           // alignment adjoint: slice-fastest projection rows with zero margins
     SliceSet set_a, set_b;
+    SliceSet set_q;          // the quads of a stack
     // autotune table: n -> schedule
     std::map<int, Tune> tune;
     std::unique_ptr<BatchPlan> plan;
@@ -361,8 +375,8 @@ void block_counts(const SliceSet &S, const SliceDev &d, int cnt[6])
 {
     cnt[0] = 0;
     cnt[G_BP] = bp_blocks(d.nx, d.ny, S.bp_rows);
-    cnt[G_TR] = tr_blocks(d.nx, d.ny);
-    cnt[G_PAD] = pad_blocks(d.ny, d.ipitch);
+    cnt[G_TR] = S.quad ? 0 : tr_blocks(d.nx, d.ny);       // k_pad_quad writes both copies
+    cnt[G_PAD] = S.quad ? pad_quad_blocks(d.ipitch, d.tpitch) : pad_blocks(d.ny, d.ipitch);
     cnt[G_EW] = ew_blocks(d.nx, d.ny);
     cnt[G_SPARE] = 0;
 }
@@ -382,6 +396,28 @@ void block_offsets(SliceSet &S)
     }
 }
 
+// Samples in the image of a ray at distance xi from the centre, averaged over
+// the angles.
+double mean_chord(const SliceDev &d, double xi)
+{
+    const double hx = 0.5 * d.nx, hy = 0.5 * d.ny, hd = std::max(hx, hy);
+    constexpr int N = 36;
+    double sum = 0.0;
+    for (int a = 0; a < N; ++a) {
+        const double th = M_PI * (a + 0.5) / N, c = std::cos(th), s = std::sin(th);
+        // the ray (xi c + t s, -xi s + t c), |t| <= D / 2, clipped to the image
+        double lo = -hd, hi = hd;
+        const double p[2] = {xi * c, -xi * s}, q[2] = {s, c}, h[2] = {hx, hy};
+        for (int k = 0; k < 2; ++k) {
+            const double t0 = (-h[k] - p[k]) / q[k], t1 = (h[k] - p[k]) / q[k];
+            lo = std::max(lo, std::min(t0, t1));
+            hi = std::min(hi, std::max(t0, t1));
+        }
+        sum += std::max(0.0, hi - lo);
+    }
+    return sum / N;
+}
+
 // Builds the per-kind logical-block maps of S (host only).
 void plan_maps(SliceSet &S)
 {
@@ -397,33 +433,52 @@ void plan_maps(SliceSet &S)
         }
         d.blk[G_FP] = 0;
     }
-    // Forward projection: a block of a slice with D samples per ray takes time
-    // a D + b, so equal block counts are not equal work.  Fitting the
-    // LDS-tiled projector's rates at D = 256 and 1024 gives b / a ~ 93 samples
-    // (the block's tile list, box loads and epilogue).  The block sequence is
-    // cut into 8 segments of equal work (a slice may straddle two), logical
-    // segment x runs on XCD x (xcd_remap), and the segments are padded to one
-    // length with empty entries.  Entries are (slice, block within the slice)
-    // pairs; slice -1 is empty.
+    // Forward projection: a block whose rays have L samples in the image takes
+    // time a L + b, so equal block counts are not equal work.  Fitting the
+    // LDS-tiled projector's rates at sides 256 and 1024 gives b / a ~ 93
+    // samples (the block's tile list, box loads and epilogue).  L is the
+    // slice's side D, and for quads the chord of the block's chunk of rays,
+    // averaged over the angles: a centre chunk's is up to twice an edge
+    // chunk's, and the segment of an XCD holds few chunks where the quads are
+    // few (8 slices of 2048^2: 1117 -> 1056 us a launch; one slice of 512^2,
+    // whose blocks all run at once, took 20.8 us for 19.8 with such weights).
+    // The block sequence is cut into 8 segments of
+    // equal work (a slice may straddle two), logical segment x runs on XCD x
+    // (xcd_remap), and the segments are padded to one length with empty
+    // entries.  Entries are (slice, block within the slice) pairs; slice -1 is
+    // empty.
     constexpr double BLOCK_COST_SAMPLES = 93.0;
     std::vector<int> cnt(n);
+    std::vector<std::vector<double>> cost(n);   // per chunk; slices of one shape share the first's
+    std::vector<int> like(n);
     double total = 0.0;
     for (int s = 0; s < n; ++s) {
         const SliceDev &d = S.h[s];
-        cnt[s] = fp_blocks(d.px, S.na, S.fp_wpb, S.fp_rays);
-        total += (double)cnt[s] * (std::max(d.nx, d.ny) + BLOCK_COST_SAMPLES);
+        cnt[s] = S.quad ? fp_quad_blocks(d.px, S.na) : fp_blocks(d.px, S.na, S.fp_wpb, S.fp_rays);
+        const SliceDev &pd = S.h[s ? like[s - 1] : 0];
+        like[s] = s > 0 && pd.nx == d.nx && pd.ny == d.ny && pd.px == d.px ? like[s - 1] : s;
+        if (S.quad && like[s] == s) {
+            const int nchunk = std::max(1, fp_blocks(d.px, 1, 4, 0));
+            for (int k = 0; k < nchunk; ++k) cost[s].push_back(mean_chord(d, (k + 0.5) * 64.0 - 0.5 * d.px) + BLOCK_COST_SAMPLES);
+        }
     }
+    auto weight = [&](int s, int b) {       // a quad's blocks are numbered chunk by chunk
+        const std::vector<double> &c = cost[like[s]];
+        if (!S.quad) return (double)std::max(S.h[s].nx, S.h[s].ny) + BLOCK_COST_SAMPLES;
+        return c[std::min(c.size() - 1, (size_t)b * c.size() / cnt[s])];
+    };
+    for (int s = 0; s < n; ++s)
+        for (int b = 0; b < cnt[s]; ++b) total += weight(s, b);
     std::vector<std::vector<std::pair<int, int>>> seg(8);
     double acc = 0.0;
     int x = 0;
-    for (int s = 0; s < n; ++s) {
-        const double w = std::max(S.h[s].nx, S.h[s].ny) + BLOCK_COST_SAMPLES;
+    for (int s = 0; s < n; ++s)
         for (int b = 0; b < cnt[s]; ++b) {
+            const double w = weight(s, b);
             while (x < 7 && acc + 0.5 * w > total * (x + 1) / 8.0) ++x;
             seg[x].push_back({s, b});
             acc += w;
         }
-    }
     size_t per = 0;
     for (const auto &v : seg) per = std::max(per, v.size());
     std::vector<int> &fm = S.hmap[G_FP];
@@ -474,9 +529,9 @@ size_t set_bytes(SliceSet &S)
 void map_signature(const SliceSet &S, std::vector<int> &sig)
 {
     sig.clear();
-    sig.reserve(5 + 4 * S.h.size());
-    sig.insert(sig.end(), {S.na, S.fp_wpb, S.fp_rays, S.fp_tile, S.bp_rows});
-    for (const SliceDev &d : S.h) sig.insert(sig.end(), {d.nx, d.ny, d.px, d.ipitch});
+    sig.reserve(6 + 5 * S.h.size());
+    sig.insert(sig.end(), {S.na, S.fp_wpb, S.fp_rays, S.fp_tile, S.bp_rows, (int)S.quad});
+    for (const SliceDev &d : S.h) sig.insert(sig.end(), {d.nx, d.ny, d.px, d.ipitch, d.tpitch});
 }
 
 ctr_status upload_set(ctr_ctx *c, SliceSet &S, char *dst = nullptr)
@@ -595,13 +650,71 @@ void fill_stack(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b)
         d.img = b.pimg ? b.pimg + (size_t)z * pimg_floats(l) : nullptr;
         d.imgT = b.pimgT ? b.pimgT + (size_t)z * pimgT_floats(l) : nullptr;
         d.rows = b.rows ? b.rows + (size_t)z * na * l.rpitch : nullptr;
-        d.prj = b.prj ? b.prj + (size_t)z * g.pa * g.px : nullptr;
-        d.src = b.src ? b.src + (size_t)z * g.nx * g.ny : nullptr;
-        d.dst = b.dst ? b.dst + (size_t)z * g.nx * g.ny : nullptr;
-        d.aux = b.aux ? b.aux + (size_t)z * g.nx * g.ny : nullptr;
+        d.prj[0] = b.prj ? b.prj + (size_t)z * g.pa * g.px : nullptr;
+        d.src[0] = b.src ? b.src + (size_t)z * g.nx * g.ny : nullptr;
+        d.dst[0] = b.dst ? b.dst + (size_t)z * g.nx * g.ny : nullptr;
+        d.aux[0] = b.aux ? b.aux + (size_t)z * g.nx * g.ny : nullptr;
         d.layer = b.layer_base + z;
+        d.nz = 1;
     }
+    S.quad = false;
     S.bp_rows = fill_rows(c, S, t.bp_rows);
+}
+
+// The descriptors of the first nz layers of a stack as quads (host only).
+void fill_quads(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b)
+{
+    const ctr_geometry &g = c->g;
+    const Layout l = make_quad_layout(g.nx, g.ny, g.px);
+    const int na = g.pa / g.ss;
+    S.fp_wpb = 4;
+    S.fp_rays = 0;
+    S.bp_rows = QBP_ROWS;
+    S.na = na;
+    S.quad = true;
+    S.h.assign((nz + QZ - 1) / QZ, SliceDev{});
+    for (size_t q = 0; q < S.h.size(); ++q) {
+        SliceDev &d = S.h[q];
+        d.nx = g.nx; d.ny = g.ny; d.px = g.px;
+        d.ipitch = l.ipitch; d.tpitch = l.tpitch; d.rpitch = l.rpitch; d.roff = l.roff;
+        d.img = b.pimg + q * quad_img_floats(l);
+        d.imgT = b.pimgT + q * quad_imgT_floats(l);
+        d.rows = b.rows + q * QZ * na * l.rpitch;
+        d.nz = std::min(QZ, nz - (int)q * QZ);
+        for (int k = 0; k < d.nz; ++k) {
+            const size_t z = q * QZ + k, plane = (size_t)g.nx * g.ny;
+            d.prj[k] = b.prj ? b.prj + z * g.pa * g.px : nullptr;
+            d.src[k] = b.src ? b.src + z * plane : nullptr;
+            d.dst[k] = b.dst ? b.dst + z * plane : nullptr;
+            d.aux[k] = b.aux ? b.aux + z * plane : nullptr;
+        }
+        d.layer = b.layer_base + (int)q * QZ;
+    }
+}
+
+// How many of n equal slices run as quads: all whole quads, and two or three
+// left over as a quad with empty places (a quad takes about two slices' time,
+// so a lone pair stays single).
+int quad_part(int n) { return n >= QZ - 1 && n % QZ >= 2 ? n : n / QZ * QZ; }
+
+// Projection blocks (over all quads of a launch) from which quads are used.  A
+// quad gives the device an eighth of the projection blocks and of the
+// backprojection threads of its four slices, so small launches lose more to
+// latency than they save in work.  Quads against single slices, us per subset:
+// 16 x 256^2, 90 angles (720 blocks) 88 / 88; 8 x 512^2, 72 (576) 104 / 118;
+// 16 x 512^2, 72 (1152) 149 / 217; 6 x 1024^2, 45 (736) 226 / 211;
+// 4 x 1024^2, 120 (960) 241 / 337; 12 x 301^2, 30 (225) 69 / 44.
+constexpr long long QUAD_MIN_BLOCKS = 900;
+
+bool quads_fill(long long fp_block_count) { return fp_block_count >= QUAD_MIN_BLOCKS; }
+
+// Layers of a uniform stack of nz that run as quads.
+int stack_quads(ctr_ctx *c, int nz)
+{
+    const ctr_geometry &g = c->g;
+    if (tuned(c, std::max(g.nx, g.ny)).fp_rays != 0) return 0;
+    const int nq = quad_part(nz);
+    return quads_fill((long long)((nq + QZ - 1) / QZ) * fp_quad_blocks(g.px, g.pa / g.ss)) ? nq : 0;
 }
 
 // Device workspace for an nz-layer stack of the current geometry.
@@ -669,7 +782,8 @@ ctr_status run_fp(ctr_ctx *c, SliceSet &S, int var, int sub, int sub_from_layer,
 {
     FpParams p{sub, c->g.ss, c->g.pa / c->g.ss, sub_from_layer, geo_power, 0};
     time_begin(c, 0);
-    launch_fp(var, S.fp_wpb, S.fp_rays, S.fp_tile, launch_of(c, S, G_FP), p, c->stream);
+    if (S.quad) launch_fp_quad(var, launch_of(c, S, G_FP), p, c->stream);
+    else launch_fp(var, S.fp_wpb, S.fp_rays, S.fp_tile, launch_of(c, S, G_FP), p, c->stream);
     POST(c, "forward projection");
     time_end(c, 0);
     return CTR_OK;
@@ -680,7 +794,8 @@ ctr_status run_bp(ctr_ctx *c, SliceSet &S, int var, int sub, int sub_from_layer,
 {
     BpParams p{sub, c->g.ss, c->g.pa / c->g.ss, c->g.pa, sub_from_layer, alpha, L, to_aux, 0, write_t};
     time_begin(c, 1);
-    launch_bp(var, S.bp_rows, launch_of(c, S, G_BP), p, c->stream);
+    if (S.quad) launch_bp_quad(var, launch_of(c, S, G_BP), p, c->stream);
+    else launch_bp(var, S.bp_rows, launch_of(c, S, G_BP), p, c->stream);
     POST(c, "backprojection");
     time_end(c, 1);
     return CTR_OK;
@@ -689,9 +804,10 @@ ctr_status run_bp(ctr_ctx *c, SliceSet &S, int var, int sub, int sub_from_layer,
 ctr_status run_kind(ctr_ctx *c, SliceSet &S, int kind)
 {
     const Launch L = launch_of(c, S, kind);
+    if (S.quad && kind == G_TR) return CTR_OK;            // launch_pad_quad wrote the transposed copy
     if (kind == G_TR) launch_transpose(L, c->stream);
-    else if (kind == G_PAD) launch_pad_in(L, c->stream);
-    else launch_unpad_out(L, c->stream);
+    else if (kind == G_PAD) S.quad ? launch_pad_quad(L, c->stream) : launch_pad_in(L, c->stream);
+    else S.quad ? launch_unpad_quad(L, c->stream) : launch_unpad_out(L, c->stream);
     POST(c, kind == G_TR ? "transpose" : (kind == G_PAD ? "pad" : "unpad"));
     return CTR_OK;
 }
@@ -946,6 +1062,55 @@ static ctr_status osem_iterations(ctr_ctx *c, SliceSet &S, int it)
     return CTR_OK;
 }
 
+// Binds the layers [z0, z0 + nz) of a stack whose parts share the workspace.
+static StackBind stack_part(const ctr_geometry &g, const StackBind &b, int z0, size_t img, size_t imgT, size_t rows)
+{
+    const size_t plane = (size_t)g.nx * g.ny;
+    StackBind o = b;
+    o.pimg = b.pimg ? b.pimg + img : nullptr;
+    o.pimgT = b.pimgT ? b.pimgT + imgT : nullptr;
+    o.rows = b.rows ? b.rows + rows : nullptr;
+    o.prj = b.prj ? b.prj + (size_t)z0 * g.pa * g.px : nullptr;
+    o.src = b.src ? b.src + (size_t)z0 * plane : nullptr;
+    o.dst = b.dst ? b.dst + (size_t)z0 * plane : nullptr;
+    o.aux = b.aux ? b.aux + (size_t)z0 * plane : nullptr;
+    o.layer_base = b.layer_base + z0;
+    return o;
+}
+
+// A stack of dN layers split into quads (set_q) and single slices (set_a),
+// either of which may be empty, with its workspace and zeroed rows.  `sets`
+// receives the parts that hold layers.
+static ctr_status split_stack(ctr_ctx *c, int dN, StackBind b, std::vector<SliceSet *> &sets)
+{
+    const ctr_geometry &g = c->g;
+    const Layout l = make_layout(g.nx, g.ny, g.px), lq = make_quad_layout(g.nx, g.ny, g.px);
+    const int na = g.pa / g.ss;
+    const int nq = stack_quads(c, dN), rest = dN - nq;
+    const size_t quads = (size_t)(nq + QZ - 1) / QZ;
+    const size_t fi = quads * quad_img_floats(lq), ft = quads * quad_imgT_floats(lq), fr = quads * QZ * na * lq.rpitch;
+    const size_t rows = fr + (size_t)rest * na * l.rpitch;
+    HIPTRY(c, c->w_pimg.ensure(sizeof(float) * (fi + (size_t)rest * pimg_floats(l))));
+    HIPTRY(c, c->w_pimgT.ensure(sizeof(float) * (ft + (size_t)rest * pimgT_floats(l))));
+    HIPTRY(c, c->w_rows.ensure(sizeof(float) * rows));
+    launch_fill(c->w_rows.f(), rows, 0.0f, c->stream);
+    POST(c, "fill rows");
+    b.pimg = c->w_pimg.f();
+    b.pimgT = c->w_pimgT.f();
+    b.rows = c->w_rows.f();
+    sets.clear();
+    if (nq > 0) {
+        fill_quads(c, c->set_q, nq, b);
+        TRY(upload_set(c, c->set_q));
+        sets.push_back(&c->set_q);
+    }
+    if (rest > 0) {
+        TRY(build_stack(c, c->set_a, rest, stack_part(g, b, nq, fi, ft, fr)));
+        sets.push_back(&c->set_a);
+    }
+    return CTR_OK;
+}
+
 // OSEM_execution, GPU.cpp:125-240: [sinogramCorrection] then for it, for k:
 // OSEM1(sub[k]) -> OSEM2(sub[k]) -> image update.
 extern "C" ctr_status ctr_osem_execution(ctr_ctx *c, float *img, float *prj, int dN, int it, int prj_correction)
@@ -954,15 +1119,14 @@ extern "C" ctr_status ctr_osem_execution(ctr_ctx *c, float *img, float *prj, int
     TRY(require_full_grid(c));
     const ctr_geometry &g = c->g;
     HIPTRY(c, hipSetDevice(c->device));
-    TRY(ensure_ws(c, dN, false, 0));
-    TRY(zero_rows(c, dN, g.pa / g.ss));
     if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     StackBind b;
-    b.pimg = c->w_pimg.f(); b.pimgT = c->w_pimgT.f(); b.rows = c->w_rows.f();
     b.prj = prj; b.src = img; b.dst = img;
-    SliceSet &S = c->set_a;
-    TRY(build_stack(c, S, dN, b));
-    return osem_iterations(c, S, it);
+    std::vector<SliceSet *> sets;
+    TRY(split_stack(c, dN, b, sets));
+    // the layers are independent: each part runs all its iterations
+    for (SliceSet *S : sets) TRY(osem_iterations(c, *S, it));
+    return CTR_OK;
 }
 
 // ctr_osem_execution with its workspace in the device array `scratch`
@@ -1700,59 +1864,88 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
         std::vector<int> order(count);
         for (int i = 0; i < count; ++i) order[i] = i;
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return slices[a].n > slices[b].n; });
+        // Runs of equal sides in that order: the part of a run that goes as
+        // quads, and the slices left.  One set of quads, and one set of single
+        // slices per distinct schedule, in the order of each schedule's
+        // largest side.
+        struct Item {
+            int at, n, quad;                   // first place in `order`, slices, held as one quad
+        };
+        std::vector<Item> items;
+        long long qblocks = 0;
+        for (int pass = 0; pass < 2; ++pass) {
+            const bool use = pass == 1 && quads_fill(qblocks);
+            items.clear();
+            for (int r = 0; r < count;) {
+                const int n = slices[order[r]].n;
+                int e = r;
+                while (e < count && slices[order[e]].n == n) ++e;
+                const int nq = tuned(c, n).fp_rays == 0 ? quad_part(e - r) : 0;
+                if (pass == 0) qblocks += (long long)((nq + QZ - 1) / QZ) * fp_quad_blocks(n, na);
+                if (use)
+                    for (int k = 0; k < nq; k += QZ) items.push_back({r + k, std::min(QZ, nq - k), 1});
+                for (int k = use ? nq : 0; k < e - r; ++k) items.push_back({r + k, 1, 0});
+                r = e;
+            }
+        }
         size_t fi = 0, ft = 0, fr = 0;
-        std::vector<Layout> lay(count);
-        for (int i = 0; i < count; ++i) {
-            lay[i] = make_layout(slices[i].n, slices[i].n, slices[i].n);
-            fi += pimg_floats(lay[i]);
-            ft += pimgT_floats(lay[i]);
-            fr += (size_t)na * lay[i].rpitch;
+        for (const Item &m : items) {
+            const int n = slices[order[m.at]].n;
+            const Layout l = m.quad ? make_quad_layout(n, n, n) : make_layout(n, n, n);
+            fi += m.quad ? quad_img_floats(l) : pimg_floats(l);
+            ft += m.quad ? quad_imgT_floats(l) : pimgT_floats(l);
+            fr += (size_t)(m.quad ? QZ : 1) * na * l.rpitch;
         }
         HIPTRY(c, P.pimg.ensure(sizeof(float) * fi));
         HIPTRY(c, P.pimgT.ensure(sizeof(float) * ft));
         HIPTRY(c, P.rows.ensure(sizeof(float) * fr));
         launch_fill(P.rows.f(), fr, 0.0f, c->stream);
         POST(c, "fill rows");
-        // one set per distinct schedule, in the order of each schedule's largest side
-        std::vector<Tune> tunes;
-        std::vector<int> set_of(count);
-        for (int r = 0; r < count; ++r) {
-            const Tune t = tuned(c, slices[order[r]].n);
+        std::vector<std::pair<Tune, bool>> kinds;
+        std::vector<int> set_of;
+        for (const Item &m : items) {
+            const Tune t = m.quad ? Tune{} : tuned(c, slices[order[m.at]].n);
             int k = 0;
-            while (k < (int)tunes.size() && !(tunes[k] == t)) ++k;
-            if (k == (int)tunes.size()) tunes.push_back(t);
-            set_of[r] = k;
-        }
-        for (const Tune &t : tunes) {
-            auto S = std::make_unique<SliceSet>();
-            S->fp_wpb = t.fp_wpb;
-            S->fp_rays = t.fp_rays;
-            S->fp_tile = t.fp_tile;
-            S->bp_rows = t.bp_rows;
-            S->na = na;
-            P.sets.push_back(std::move(S));
+            while (k < (int)kinds.size() && !(kinds[k].first == t && kinds[k].second == (m.quad != 0))) ++k;
+            if (k == (int)kinds.size()) {
+                kinds.push_back({t, m.quad != 0});
+                auto S = std::make_unique<SliceSet>();
+                S->fp_wpb = t.fp_wpb;
+                S->fp_rays = t.fp_rays;
+                S->fp_tile = t.fp_tile;
+                S->bp_rows = m.quad ? QBP_ROWS : t.bp_rows;
+                S->quad = m.quad != 0;
+                S->na = na;
+                P.sets.push_back(std::move(S));
+            }
+            set_of.push_back(k);
         }
         size_t oi = 0, ot = 0, orr = 0;
-        for (int r = 0; r < count; ++r) {
-            const int i = order[r];
-            const Layout &l = lay[i];
+        for (size_t q = 0; q < items.size(); ++q) {
+            const Item &m = items[q];
+            const int n = slices[order[m.at]].n;
+            const Layout l = m.quad ? make_quad_layout(n, n, n) : make_layout(n, n, n);
             SliceDev d{};
-            d.nx = d.ny = d.px = slices[i].n;
+            d.nx = d.ny = d.px = n;
             d.ipitch = l.ipitch; d.tpitch = l.tpitch; d.rpitch = l.rpitch; d.roff = l.roff;
             d.img = P.pimg.f() + oi;
             d.imgT = P.pimgT.f() + ot;
             d.rows = P.rows.f() + orr;
-            d.prj = slices[i].prj;
-            d.src = slices[i].img;
-            d.dst = slices[i].img;
-            d.layer = r;
-            P.sets[set_of[r]]->h.push_back(d);
-            oi += pimg_floats(l);
-            ot += pimgT_floats(l);
-            orr += (size_t)na * l.rpitch;
+            d.nz = m.n;
+            for (int k = 0; k < m.n; ++k) {
+                const ctr_slice &sl = slices[order[m.at + k]];
+                d.prj[k] = sl.prj;
+                d.src[k] = sl.img;
+                d.dst[k] = sl.img;
+            }
+            d.layer = m.at;
+            P.sets[set_of[q]]->h.push_back(d);
+            oi += m.quad ? quad_img_floats(l) : pimg_floats(l);
+            ot += m.quad ? quad_imgT_floats(l) : pimgT_floats(l);
+            orr += (size_t)(m.quad ? QZ : 1) * na * l.rpitch;
         }
         for (auto &S : P.sets) {
-            S->bp_rows = fill_rows(c, *S, S->bp_rows);
+            if (!S->quad) S->bp_rows = fill_rows(c, *S, S->bp_rows);
             TRY(upload_set(c, *S));
         }
     }
@@ -1917,7 +2110,8 @@ extern "C" ctr_status ctr_autotune(ctr_ctx *c, int n, ctr_schedule *best_out)
         float *base = mem.f() + f_slice * k;
         d.nx = d.ny = d.px = n;
         d.ipitch = l.ipitch; d.tpitch = l.tpitch; d.rpitch = l.rpitch; d.roff = l.roff;
-        d.img = base; d.imgT = base + f_img; d.rows = base + f_img + f_imgT; d.prj = base + f_img + f_imgT + f_rows;
+        d.img = base; d.imgT = base + f_img; d.rows = base + f_img + f_imgT; d.prj[0] = base + f_img + f_imgT + f_rows;
+        d.nz = 1;
     }
     hipEvent_t e0, e1;
     HIPTRY(c, hipEventCreate(&e0));

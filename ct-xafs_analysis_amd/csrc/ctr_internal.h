@@ -28,18 +28,27 @@ constexpr int PAD = 100;
 // per lane of a wave); larger slices use the direct-gather projector.
 constexpr int LDS_FP_MAX_SIDE = 60 * 64;
 
+// Quads: four slices of one geometry held interleaved.  A texel of img / imgT
+// and an entry of rows is then the four slices' values side by side (16
+// bytes), the pitches count texels, and the frame is QPAD texels wide.  One
+// coordinate, bin or address serves all four slices.
+constexpr int QZ = 4;
+constexpr int QPAD = 96;
+
 struct SliceDev {
-    float *img;          // padded image (pitch ipitch, ny + 2 PAD rows)
+    float *img;          // padded image (pitch ipitch, ny + 2 PAD rows; QPAD for a quad)
     float *imgT;         // padded transposed image (pitch tpitch, nx + 2 PAD rows)
-    const float *prj;    // sinogram [pa][px], unpadded
     float *rows;         // compact subset rows [pa/ss][rpitch], bin b at entry roff + b
-    const float *src;    // unpadded [ny][nx] source of pad_in
-    float *dst;          // unpadded [ny][nx] destination of unpad_out
-    float *aux;          // unpadded [ny][nx] output plane of to_aux backprojections
+    // one entry per slice: entry 0 of a single slice, entries 0 .. nz - 1 of a quad
+    const float *prj[QZ];    // sinogram [pa][px], unpadded
+    const float *src[QZ];    // unpadded [ny][nx] source of pad_in
+    float *dst[QZ];          // unpadded [ny][nx] destination of unpad_out
+    float *aux[QZ];          // unpadded [ny][nx] output plane of to_aux backprojections
     int nx, ny, px;
     int ipitch, tpitch, rpitch;
     int roff;            // zeros before bin 0 (and at least as many after bin px - 1) in a row
     int layer;           // index in its stack (subset index for the power iteration)
+    int nz;              // slices held: 1, or 1 .. QZ in a quad (the rest of a quad stays zero)
     int blk[6];          // first logical block of this slice for each grid kind (the
                          // G_FP map holds (slice, block) pairs instead)
 };
@@ -76,6 +85,13 @@ struct BpParams {
 // ---- launchers (ctr_kernels.hip) ----
 void launch_fp(int var, int wpb, int rays, int tile, const Launch &L, const FpParams &p, hipStream_t stream);
 void launch_bp(int var, int rows, const Launch &L, const BpParams &p, hipStream_t stream);
+// The same over quads (a set of quads only; LDS-tiled projector).
+void launch_fp_quad(int var, const Launch &L, const FpParams &p, hipStream_t stream);
+void launch_bp_quad(int var, const Launch &L, const BpParams &p, hipStream_t stream);
+void launch_pad_quad(const Launch &L, hipStream_t stream);     // src planes -> both padded copies
+void launch_unpad_quad(const Launch &L, hipStream_t stream);
+// Rows per backprojection thread of a quad.
+constexpr int QBP_ROWS = 4;
 void launch_transpose(const Launch &L, hipStream_t stream);
 void launch_pad_in(const Launch &L, hipStream_t stream);
 void launch_unpad_out(const Launch &L, hipStream_t stream);
@@ -138,8 +154,10 @@ void launch_align_grad(const float *pimg, const float *pimgT, int ipitch, int tp
 
 // blocks per slice for each grid kind
 int fp_blocks(int px, int na, int wpb, int rays);
+int fp_quad_blocks(int px, int na);
 int bp_blocks(int nx, int ny, int rows);
 int tr_blocks(int nx, int ny);
+int pad_quad_blocks(int ipitch, int tpitch);
 int pad_blocks(int ny, int ipitch);
 int ew_blocks(int nx, int ny);
 size_t l2_partial_count(int nz);
