@@ -1258,16 +1258,24 @@ extern "C" ctr_status ctr_fbp_execution(ctr_ctx *c, float *img, float *prj, int 
     HIPTRY(c, hipSetDevice(c->device));
     TRY(twiddles(c, g.zp));
     const Layout l = make_layout(g.nx, g.ny, g.px);
-    HIPTRY(c, c->w_rows.ensure(sizeof(float) * (size_t)dN * g.pa * l.rpitch));
-    launch_fill(c->w_rows.f(), (size_t)dN * g.pa * l.rpitch, 0.0f, c->stream);
-    POST(c, "fill rows");
+    // whole quads of layers (and two or three left over) filter and
+    // backproject interleaved, the others singly
+    int nq = quad_part(dN);
+    if ((long long)((nq + QZ - 1) / QZ) * fbp_quad_blocks(g.nx, g.ny) < FBP_QUAD_MIN_BLOCKS || g.zp > FBP_QUAD_MAX_ZP) nq = 0;
+    const size_t qrows = (size_t)((nq + QZ - 1) / QZ) * QZ, row = (size_t)g.pa * l.rpitch;
+    HIPTRY(c, c->w_rows.ensure(sizeof(float) * (qrows + (size_t)(dN - nq)) * row));
     if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
-    launch_fbp_filter(prj, c->w_rows.f(), dN, g.pa, g.px, l.rpitch, l.roff, g.zp,
-                      static_cast<const float2 *>(c->tw.p), c->stream);
-    POST(c, "FBP filter");
-    launch_fbp_bp(c->w_rows.f(), img, static_cast<const float2 *>(c->cs.p), dN, g.nx, g.ny, g.pa, g.px, l.rpitch,
-                  l.roff, c->stream);
-    POST(c, "backProjectionFBP");
+    for (int part = 0; part < 2; ++part) {
+        const int z0 = part == 0 ? 0 : nq, nz = part == 0 ? nq : dN - nq, quads = part == 0;
+        if (nz == 0) continue;
+        float *rows = c->w_rows.f() + (part == 0 ? 0 : qrows * row);
+        launch_fbp_filter(prj + (size_t)z0 * g.pa * g.px, rows, nz, g.pa, g.px, l.rpitch, l.roff, g.zp,
+                          static_cast<const float2 *>(c->tw.p), quads, c->stream);
+        POST(c, "FBP filter");
+        launch_fbp_bp(rows, img + (size_t)z0 * g.nx * g.ny, static_cast<const float2 *>(c->cs.p), nz, g.nx, g.ny, g.pa,
+                      g.px, l.rpitch, l.roff, quads, c->stream);
+        POST(c, "backProjectionFBP");
+    }
     return CTR_OK;
 }
 
@@ -1731,10 +1739,8 @@ extern "C" ctr_status ctr_op_fbp_filter(ctr_ctx *c, const float *prj, float *fpr
     TRY(twiddles(c, g.zp));
     const Layout l = make_layout(g.nx, g.ny, g.px);
     HIPTRY(c, c->w_rows.ensure(sizeof(float) * (size_t)dN * g.pa * l.rpitch));
-    launch_fill(c->w_rows.f(), (size_t)dN * g.pa * l.rpitch, 0.0f, c->stream);
-    POST(c, "fill rows");
     launch_fbp_filter(prj, c->w_rows.f(), dN, g.pa, g.px, l.rpitch, l.roff, g.zp,
-                      static_cast<const float2 *>(c->tw.p), c->stream);
+                      static_cast<const float2 *>(c->tw.p), 0, c->stream);
     POST(c, "FBP filter");
     // all rows are "subset 0 of 1": copy the padded rows back out
     launch_rows_to_full(c->w_rows.f(), fprj, dN, g.pa, l.rpitch, l.roff, g.pa, g.px, 0, 1, c->stream);
@@ -1753,7 +1759,7 @@ extern "C" ctr_status ctr_op_fbp_backprojection(ctr_ctx *c, const float *fprj, f
     launch_full_to_rows(fprj, c->w_rows.f(), dN, g.pa, l.rpitch, l.roff, g.pa, g.px, 0, 1, c->stream);
     POST(c, "full to rows");
     launch_fbp_bp(c->w_rows.f(), img, static_cast<const float2 *>(c->cs.p), dN, g.nx, g.ny, g.pa, g.px, l.rpitch,
-                  l.roff, c->stream);
+                  l.roff, 0, c->stream);
     POST(c, "backProjectionFBP");
     return CTR_OK;
 }

@@ -129,9 +129,14 @@ void launch_focus_index(const float *img, int nz, int nx, int ny, const float *s
 void launch_power3(const float *cnd, const float *l2, float *pimg, int nz, int nx, int ny, int ipitch,
                    hipStream_t stream);
 void launch_fbp_filter(const float *prj, float *frows, int nz, int pa, int px, int rpitch, int roff, int zp,
-                       const float2 *tw, hipStream_t stream);
+                       const float2 *tw, int quads, hipStream_t stream);
+// Blocks of 64 x 4 pixels from which layers run FBP as quads (8 slices of
+// 256^2, 360 angles: 98 us as quads, 106 singly).
+constexpr long long FBP_QUAD_MIN_BLOCKS = 512;
+// A quad's filter block holds two transforms (16 ZP bytes of LDS).
+constexpr int FBP_QUAD_MAX_ZP = 4096;
 void launch_fbp_bp(const float *frows, float *img, const float2 *cs, int nz, int nx, int ny, int pa,
-                   int px, int rpitch, int roff, hipStream_t stream);
+                   int px, int rpitch, int roff, int quads, hipStream_t stream);
 void launch_rows_to_full(const float *rows, float *full, int nz, int na, int rpitch, int roff, int pa, int px,
                          int sub, int ss, hipStream_t stream);
 void launch_full_to_rows(const float *full, float *rows, int nz, int na, int rpitch, int roff, int pa, int px,
@@ -155,6 +160,7 @@ void launch_align_grad(const float *pimg, const float *pimgT, int ipitch, int tp
 // blocks per slice for each grid kind
 int fp_blocks(int px, int na, int wpb, int rays);
 int fp_quad_blocks(int px, int na);
+int fbp_quad_blocks(int nx, int ny);
 int bp_blocks(int nx, int ny, int rows);
 int tr_blocks(int nx, int ny);
 int pad_quad_blocks(int ipitch, int tpitch);

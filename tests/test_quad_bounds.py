@@ -210,3 +210,23 @@ def test_backprojector_segments(nx, ny, px):
                 assert (b >= lo[:, None, None]).all() and (b <= hi[:, None, None]).all()
                 assert (hi - lo + 1).max() <= QBP_SEG
                 assert lo.min() + l.roff >= 0 and hi.max() + l.roff < l.rpitch
+
+
+@pytest.mark.parametrize("rows,seg", [(4, 72), (8, 72), (16, 72)])
+@pytest.mark.parametrize("n,px", [(1024, 1024), (37, 41), (300, 128)])
+def test_fbp_segments_hold_every_bin(n, px, rows, seg):
+    """The staged bins of a block of 64 columns, from the lowest corner's bin to
+    the highest one's right neighbour (float32, the kernel's operations)."""
+    rng = np.random.default_rng(n)
+    th = np.concatenate([np.linspace(0, 2 * np.pi, 181), rng.uniform(0, 2 * np.pi, 60)])
+    C, S = np.cos(th).astype(f32)[:, None, None], np.sin(th).astype(f32)[:, None, None]
+    tiles = [(x, y) for x in range((n + 63) // 64) for y in range((n + rows - 1) // rows)]
+    for tx, ty in [tiles[0], tiles[-1]] + [tiles[i] for i in rng.integers(0, len(tiles), 12)]:
+        X = np.minimum(tx * 64 + np.arange(64), n - 1).astype(f32) - f32(n * 0.5)
+        Y = np.minimum(ty * rows + np.arange(rows), n - 1).astype(f32) - f32(n * 0.5)
+        u = (((X[None, None, :] * C).astype(f32) - (Y[None, :, None] * S).astype(f32)).astype(f32) + f32(px * 0.5)).astype(f32)
+        b = np.floor(u)
+        lo = b[:, [0, 0, -1, -1], [0, -1, 0, -1]].min(1)
+        hi = b[:, [0, 0, -1, -1], [0, -1, 0, -1]].max(1)
+        assert (b >= lo[:, None, None]).all() and (b <= hi[:, None, None]).all()
+        assert (hi - lo + 2).max() <= seg
