@@ -1170,6 +1170,33 @@ extern "C" ctr_status ctr_osem_execution_noalloc(ctr_ctx *c, float *img, float *
     return osem_iterations(c, S, it);
 }
 
+// The prox of the stack v of dN layers into the images of one of its parts.
+static ctr_status run_tv(ctr_ctx *c, SliceSet &S, int fista, const float *v, int dN, int sub)
+{
+    const SliceDev &d = S.h[0];
+    const Layout l = S.quad ? make_quad_layout(d.nx, d.ny, d.px) : make_layout(d.nx, d.ny, d.px);
+    TvPad t{};
+    t.v = v;
+    t.pimg = d.img;
+    t.pimgT = d.imgT;
+    t.ifl = S.quad ? quad_img_floats(l) : pimg_floats(l);
+    t.tfl = S.quad ? quad_imgT_floats(l) : pimgT_floats(l);
+    t.ipitch = d.ipitch;
+    t.tpitch = d.tpitch;
+    t.z0 = d.layer;
+    for (const SliceDev &e : S.h) t.n += e.nz;
+    t.nz = dN;
+    t.nx = d.nx;
+    t.ny = d.ny;
+    t.fista = fista;
+    t.sub = sub;
+    t.L = c->w_l2.f();
+    t.lambda_fista = (double)c->g.cs_lambda;
+    launch_tv_pad(S.quad, t, c->stream);
+    POST(c, fista ? "FISTA3D" : "ISTA3D");
+    return CTR_OK;
+}
+
 // FISTA_OSEM_execution, GPU.cpp:243-405.  L2norm is filled with 0.5
 // (GPU.cpp:326), so lambda = CSlambda.  First sub-iteration: ISTA3D of the
 // pre-update image replaces the OS-EM result (GPU.cpp:329-330, 369-377);
@@ -1183,34 +1210,32 @@ extern "C" ctr_status ctr_fista_osem_execution(ctr_ctx *c, float *img, float *pr
     TRY(require_full_grid(c));
     const ctr_geometry &g = c->g;
     HIPTRY(c, hipSetDevice(c->device));
-    TRY(ensure_ws(c, dN, false, 1));
+    HIPTRY(c, c->w_aux1.ensure(sizeof(float) * (size_t)dN * g.nx * g.ny));
     HIPTRY(c, c->w_l2.ensure(sizeof(float) * g.ss));
-    TRY(zero_rows(c, dN, g.pa / g.ss));
     launch_fill(c->w_l2.f(), g.ss, 0.5f, c->stream);
     POST(c, "fill L2norm");
     if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
-    const Layout l = make_layout(g.nx, g.ny, g.px);
     StackBind b;
-    b.pimg = c->w_pimg.f(); b.pimgT = c->w_pimgT.f(); b.rows = c->w_rows.f();
     b.prj = prj; b.src = img; b.dst = img; b.aux = c->w_aux1.f();
-    SliceSet &S = c->set_a;
-    TRY(build_stack(c, S, dN, b));
-    TRY(run_kind(c, S, G_PAD));
+    std::vector<SliceSet *> sets;
+    TRY(split_stack(c, dN, b, sets));
+    for (SliceSet *S : sets) {
+        TRY(run_kind(c, *S, G_PAD));
+        TRY(run_kind(c, *S, G_TR));
+    }
     bool first = true;
     for (int i = 0; i < it; ++i)
         for (int k = 0; k < g.ss; ++k) {
-            TRY(run_kind(c, S, G_TR));
-            TRY(run_fp(c, S, FP_RATIO, c->sub[k], 0, 0));
-            TRY(run_bp(c, S, BP_OSEM2, c->sub[k], 0, 0.0f, nullptr, 1));
+            for (SliceSet *S : sets) {
+                TRY(run_fp(c, *S, FP_RATIO, c->sub[k], 0, 0));
+                TRY(run_bp(c, *S, BP_OSEM2, c->sub[k], 0, 0.0f, nullptr, 1));
+            }
             // the prox reads an unpadded stack: the initial image (first step,
             // still in the caller's buffer) or the OS-EM update (aux)
-            const float *v = first ? img : c->w_aux1.f();
-            launch_tv(first ? 0 : 1, nullptr, v, nullptr, nullptr, c->w_pimg.f(), nullptr, 1, l.ipitch, dN, g.nx,
-                      g.ny, c->w_l2.f(), c->sub[k], (double)g.cs_lambda, c->stream);
-            POST(c, first ? "ISTA3D" : "FISTA3D");
+            for (SliceSet *S : sets) TRY(run_tv(c, *S, first ? 0 : 1, first ? img : c->w_aux1.f(), dN, c->sub[k]));
             first = false;
         }
-    TRY(run_kind(c, S, G_EW));
+    for (SliceSet *S : sets) TRY(run_kind(c, *S, G_EW));
     return CTR_OK;
 }
 
@@ -1223,24 +1248,24 @@ extern "C" ctr_status ctr_aart_execution(ctr_ctx *c, float *img, float *prj, int
     TRY(require_full_grid(c));
     const ctr_geometry &g = c->g;
     HIPTRY(c, hipSetDevice(c->device));
-    TRY(ensure_ws(c, dN, false, 0));
-    TRY(zero_rows(c, dN, g.pa / g.ss));
     if (g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     const float alpha = (g.mode == 3) ? g.wt2 : g.wt1;   // GPU.cpp:1161-1165
     StackBind b;
-    b.pimg = c->w_pimg.f(); b.pimgT = c->w_pimgT.f(); b.rows = c->w_rows.f();
     b.prj = prj; b.src = img; b.dst = img;
-    SliceSet &S = c->set_a;
-    TRY(build_stack(c, S, dN, b));
-    TRY(run_kind(c, S, G_PAD));   // zero borders (the interior is overwritten next)
-    TRY(run_bp(c, S, BP_INIT, c->sub[0], 0, 0.0f, nullptr, 0));
-    for (int i = 0; i < it; ++i)
-        for (int k = 0; k < g.ss; ++k) {
-            TRY(run_kind(c, S, G_TR));
-            TRY(run_fp(c, S, FP_RESID, c->sub[k], 0, 0));
-            TRY(run_bp(c, S, BP_AART2, c->sub[k], 0, alpha, nullptr, 0));
-        }
-    TRY(run_kind(c, S, G_EW));
+    std::vector<SliceSet *> sets;
+    TRY(split_stack(c, dN, b, sets));
+    for (SliceSet *S : sets) {
+        // zero borders of both copies (the interior is overwritten next)
+        TRY(run_kind(c, *S, G_PAD));
+        TRY(run_kind(c, *S, G_TR));
+        TRY(run_bp(c, *S, BP_INIT, c->sub[0], 0, 0.0f, nullptr, 0, 1));
+        for (int i = 0; i < it; ++i)
+            for (int k = 0; k < g.ss; ++k) {
+                TRY(run_fp(c, *S, FP_RESID, c->sub[k], 0, 0));
+                TRY(run_bp(c, *S, BP_AART2, c->sub[k], 0, alpha, nullptr, 0, 1));
+            }
+        TRY(run_kind(c, *S, G_EW));
+    }
     return CTR_OK;
 }
 

@@ -102,6 +102,20 @@ void launch_sino_correction(const float *src, float *dst, const float2 *cs_corr,
 void launch_tv(int fista, const float *x, const float *v, const float *b, float *w_new, float *x_new,
                float *b_new, int out_padded, int ipitch, int nz, int nx, int ny, const float *L,
                int sub, double lambda_fista, hipStream_t stream);
+// The prox of the layers [z0, z0 + n) of the unpadded stack v of nz layers,
+// into the padded images of a set (quads or single slices, one after another
+// every ifl floats) and their transposed copies (every tfl floats).
+struct TvPad {
+    const float *v;
+    float *pimg, *pimgT;
+    size_t ifl, tfl;
+    int ipitch, tpitch, z0, n, nz, nx, ny, fista, sub;
+    const float *L;
+    double lambda_fista;
+    long long nblk;
+};
+constexpr int TV_R = 4;                  // rows per thread
+void launch_tv_pad(bool quad, TvPad t, hipStream_t stream);
 void launch_tv2d(const float *v, float *x_new, int nz, int nx, int ny, float lambda, float lower,
                  hipStream_t stream);
 void launch_l2(const float *src, int nz, size_t n, float *partial, float *l2, hipStream_t stream);
