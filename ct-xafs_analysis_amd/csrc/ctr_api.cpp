@@ -679,7 +679,7 @@ void fill_quads(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b)
         d.ipitch = l.ipitch; d.tpitch = l.tpitch; d.rpitch = l.rpitch; d.roff = l.roff;
         d.img = b.pimg + q * quad_img_floats(l);
         d.imgT = b.pimgT + q * quad_imgT_floats(l);
-        d.rows = b.rows + q * QZ * na * l.rpitch;
+        d.rows = b.rows ? b.rows + q * QZ * na * l.rpitch : nullptr;
         d.nz = std::min(QZ, nz - (int)q * QZ);
         for (int k = 0; k < d.nz; ++k) {
             const size_t z = q * QZ + k, plane = (size_t)g.nx * g.ny;
@@ -703,18 +703,27 @@ int quad_part(int n) { return n >= QZ - 1 && n % QZ >= 2 ? n : n / QZ * QZ; }
 // latency than they save in work.  Quads against single slices, us per subset:
 // 16 x 256^2, 90 angles (720 blocks) 88 / 88; 8 x 512^2, 72 (576) 104 / 118;
 // 16 x 512^2, 72 (1152) 149 / 217; 6 x 1024^2, 45 (736) 226 / 211;
-// 4 x 1024^2, 120 (960) 241 / 337; 12 x 301^2, 30 (225) 69 / 44.
+// 4 x 1024^2, 120 (960) 241 / 337; 12 x 301^2, 30 (225) 69 / 44.  The alignment
+// forward with its derivative, near the line: 4 x 128^2, 900 angles (900) 81 / 96;
+// 4 x 512^2, 225 (904) 163 / 184; 3 x 256^2, 450 (900) 98 / 104; 4 x 1024^2, 113
+// (912) 311 / 307.
 constexpr long long QUAD_MIN_BLOCKS = 900;
 
 bool quads_fill(long long fp_block_count) { return fp_block_count >= QUAD_MIN_BLOCKS; }
 
-// Layers of a uniform stack of nz that run as quads.
+// Layers of nz equal ones that a projection of na angles takes as quads.
+int launch_quads(int nz, int px, int na)
+{
+    const int nq = quad_part(nz);
+    return quads_fill((long long)((nq + QZ - 1) / QZ) * fp_quad_blocks(px, na)) ? nq : 0;
+}
+
+// Layers of a uniform stack of nz that the subset drivers run as quads.
 int stack_quads(ctr_ctx *c, int nz)
 {
     const ctr_geometry &g = c->g;
     if (tuned(c, std::max(g.nx, g.ny)).fp_rays != 0) return 0;
-    const int nq = quad_part(nz);
-    return quads_fill((long long)((nq + QZ - 1) / QZ) * fp_quad_blocks(g.px, g.pa / g.ss)) ? nq : 0;
+    return launch_quads(nz, g.px, g.pa / g.ss);
 }
 
 // Device workspace for an nz-layer stack of the current geometry.
@@ -1078,26 +1087,28 @@ static StackBind stack_part(const ctr_geometry &g, const StackBind &b, int z0, s
     return o;
 }
 
-// A stack of dN layers split into quads (set_q) and single slices (set_a),
-// either of which may be empty, with its workspace and zeroed rows.  `sets`
-// receives the parts that hold layers.
-static ctr_status split_stack(ctr_ctx *c, int dN, StackBind b, std::vector<SliceSet *> &sets)
+// A stack of dN layers split into quads (set_q, the first nq layers) and single
+// slices (set_a), either of which may be empty, with its workspace: the padded
+// images and, with_rows, zeroed subset rows.  `sets` receives
+// the parts that hold layers.
+static ctr_status split_stack(ctr_ctx *c, int dN, int nq, bool with_rows, StackBind b, std::vector<SliceSet *> &sets)
 {
     const ctr_geometry &g = c->g;
     const Layout l = make_layout(g.nx, g.ny, g.px), lq = make_quad_layout(g.nx, g.ny, g.px);
-    const int na = g.pa / g.ss;
-    const int nq = stack_quads(c, dN), rest = dN - nq;
+    const int na = with_rows ? g.pa / g.ss : 0, rest = dN - nq;
     const size_t quads = (size_t)(nq + QZ - 1) / QZ;
     const size_t fi = quads * quad_img_floats(lq), ft = quads * quad_imgT_floats(lq), fr = quads * QZ * na * lq.rpitch;
     const size_t rows = fr + (size_t)rest * na * l.rpitch;
     HIPTRY(c, c->w_pimg.ensure(sizeof(float) * (fi + (size_t)rest * pimg_floats(l))));
     HIPTRY(c, c->w_pimgT.ensure(sizeof(float) * (ft + (size_t)rest * pimgT_floats(l))));
-    HIPTRY(c, c->w_rows.ensure(sizeof(float) * rows));
-    launch_fill(c->w_rows.f(), rows, 0.0f, c->stream);
-    POST(c, "fill rows");
+    if (with_rows) {
+        HIPTRY(c, c->w_rows.ensure(sizeof(float) * rows));
+        launch_fill(c->w_rows.f(), rows, 0.0f, c->stream);
+        POST(c, "fill rows");
+        b.rows = c->w_rows.f();
+    }
     b.pimg = c->w_pimg.f();
     b.pimgT = c->w_pimgT.f();
-    b.rows = c->w_rows.f();
     sets.clear();
     if (nq > 0) {
         fill_quads(c, c->set_q, nq, b);
@@ -1123,7 +1134,7 @@ extern "C" ctr_status ctr_osem_execution(ctr_ctx *c, float *img, float *prj, int
     StackBind b;
     b.prj = prj; b.src = img; b.dst = img;
     std::vector<SliceSet *> sets;
-    TRY(split_stack(c, dN, b, sets));
+    TRY(split_stack(c, dN, stack_quads(c, dN), true, b, sets));
     // the layers are independent: each part runs all its iterations
     for (SliceSet *S : sets) TRY(osem_iterations(c, *S, it));
     return CTR_OK;
@@ -1218,7 +1229,7 @@ extern "C" ctr_status ctr_fista_osem_execution(ctr_ctx *c, float *img, float *pr
     StackBind b;
     b.prj = prj; b.src = img; b.dst = img; b.aux = c->w_aux1.f();
     std::vector<SliceSet *> sets;
-    TRY(split_stack(c, dN, b, sets));
+    TRY(split_stack(c, dN, stack_quads(c, dN), true, b, sets));
     for (SliceSet *S : sets) {
         TRY(run_kind(c, *S, G_PAD));
         TRY(run_kind(c, *S, G_TR));
@@ -1253,7 +1264,7 @@ extern "C" ctr_status ctr_aart_execution(ctr_ctx *c, float *img, float *prj, int
     StackBind b;
     b.prj = prj; b.src = img; b.dst = img;
     std::vector<SliceSet *> sets;
-    TRY(split_stack(c, dN, b, sets));
+    TRY(split_stack(c, dN, stack_quads(c, dN), true, b, sets));
     for (SliceSet *S : sets) {
         // zero borders of both copies (the interior is overwritten next)
         TRY(run_kind(c, *S, G_PAD));
@@ -2251,12 +2262,29 @@ ctr_status align_forward(ctr_ctx *c, const float *img, const float *shifts, floa
 {
     TRY(op_prologue(c, img, prj, dN));
     if (!std::isfinite(center)) return fail(c, CTR_INVALID_ARGUMENT, "center is not finite");
-    TRY(align_pad(c, img, dN));
     const ctr_geometry &g = c->g;
-    const Layout l = make_layout(g.nx, g.ny, g.px);
-    launch_align_forward(c->w_pimg.f(), c->w_pimgT.f(), l.ipitch, l.tpitch, static_cast<const float2 *>(c->cs.p),
-                         shifts, center, prj, dprj, dN, g.nx, g.ny, g.pa, g.px, c->stream);
-    POST(c, "align forward");
+    StackBind b;
+    b.src = img;
+    std::vector<SliceSet *> sets;
+    const int nq = std::max(g.nx, g.ny) <= LDS_FP_MAX_SIDE ? launch_quads(dN, g.px, g.pa) : 0;
+    TRY(split_stack(c, dN, nq, false, b, sets));
+    for (SliceSet *S : sets) {
+        TRY(run_kind(c, *S, G_PAD));
+        TRY(run_kind(c, *S, G_TR));
+        const SliceDev &d = S->h[0];
+        const size_t o = (size_t)d.layer * g.pa * g.px;
+        const float2 *cs = static_cast<const float2 *>(c->cs.p);
+        float *out = prj + o, *dout = dprj ? dprj + o : nullptr;
+        if (S->quad) {
+            const Layout l = make_quad_layout(g.nx, g.ny, g.px);
+            launch_align_quad(d.img, d.imgT, quad_img_floats(l), quad_imgT_floats(l), d.ipitch, d.tpitch, cs, shifts,
+                              center, out, dout, nq, g.nx, g.ny, g.pa, g.px, c->stream);
+        } else {
+            launch_align_forward(d.img, d.imgT, d.ipitch, d.tpitch, cs, shifts, center, out, dout, dN - nq, g.nx, g.ny,
+                                 g.pa, g.px, c->stream);
+        }
+        POST(c, "align forward");
+    }
     return CTR_OK;
 }
 

@@ -160,6 +160,11 @@ void launch_full_to_rows(const float *full, float *rows, int nz, int na, int rpi
 void launch_align_forward(const float *pimg, const float *pimgT, int ipitch, int tpitch, const float2 *cs,
                           const float *shifts, float center, float *prj, float *dprj, int nz, int nx, int ny, int pa,
                           int px, hipStream_t stream);
+// The same over nz layers as quads, whose padded copies follow one another
+// every ifl and tfl floats.  Needs sides of at most LDS_FP_MAX_SIDE.
+void launch_align_quad(const float *img, const float *imgT, size_t ifl, size_t tfl, int ipitch, int tpitch,
+                       const float2 *cs, const float *shifts, float center, float *prj, float *dprj, int nz, int nx,
+                       int ny, int pa, int px, hipStream_t stream);
 // Zero rays on either side of each projection row in the adjoint's copy of
 // the rows, and that copy's size in floats (slice-fastest, in chunks of 1, 4
 // or 16 slices).
