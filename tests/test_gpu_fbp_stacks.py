@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("n,px,pa,zp,dn", [
     (2, 2, 3, 2, 1), (3, 3, 5, 4, 2), (8, 8, 5, 8, 1), (20, 17, 7, 32, 5),
-    (129, 100, 23, 128, 3),       # one row per block, an odd angle count
+    (129, 100, 23, 128, 3),       # 4 split rows per block, an odd angle count
     (300, 390, 41, 512, 3),       # 8 rows per block
     (257, 257, 24, 1024, 20),     # quads of 4 rows per block
     (300, 260, 40, 512, 35),      # quads of 16 rows per block, the last with three layers
