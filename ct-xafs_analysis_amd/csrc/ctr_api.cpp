@@ -605,15 +605,17 @@ struct StackBind {
 void fill_stack(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b);
 
 // Rows per backprojection thread for the slices of S: the side's schedule
-// (rows), halved while the launch would give the device fewer than 4 blocks
+// (rows), halved while the launch would give the device fewer than 3.5 blocks
 // per compute unit (unless the context runs every stack as scheduled).  One
-// slice of 512^2 at 8 rows is 128 blocks; at 1 row, 1024.  Every row count
-// gives each pixel the same sum in the same order, so only the launch shape
+// slice of 512^2 at 8 rows is 128 blocks; at 1 row, 1024.  Five 301^2 (950 blocks
+// at 2 rows, 1900 at 1) take 11.7 us at 2 and 13.4 at 1, two 700^2 (968 at 4) 22.1
+// at 4 and 25.3 at 2, six 512^2 (768 at 8) 33.1 at 8 and 31.8 at 4.  Every row
+// count gives each pixel the same sum in the same order, so only the launch shape
 // changes.
 int fill_rows(const ctr_ctx *c, const SliceSet &S, int rows)
 {
     if (!c->adaptive_rows) return rows;
-    const long long want = 4LL * c->cus;
+    const long long want = 7LL * c->cus / 2;
     auto blocks = [&](int r) {
         long long n = 0;
         for (const SliceDev &d : S.h) n += bp_blocks(d.nx, d.ny, r);
@@ -697,25 +699,30 @@ void fill_quads(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b)
 // so a lone pair stays single).
 int quad_part(int n) { return n >= QZ - 1 && n % QZ >= 2 ? n : n / QZ * QZ; }
 
-// Projection blocks (over all quads of a launch) from which quads are used.  A
-// quad gives the device an eighth of the projection blocks and of the
-// backprojection threads of its four slices, so small launches lose more to
-// latency than they save in work.  Quads against single slices, us per subset:
-// 16 x 256^2, 90 angles (720 blocks) 88 / 88; 8 x 512^2, 72 (576) 104 / 118;
-// 16 x 512^2, 72 (1152) 149 / 217; 6 x 1024^2, 45 (736) 226 / 211;
-// 4 x 1024^2, 120 (960) 241 / 337; 12 x 301^2, 30 (225) 69 / 44.  The alignment
-// forward with its derivative, near the line: 4 x 128^2, 900 angles (900) 81 / 96;
-// 4 x 512^2, 225 (904) 163 / 184; 3 x 256^2, 450 (900) 98 / 104; 4 x 1024^2, 113
-// (912) 311 / 307.
-constexpr long long QUAD_MIN_BLOCKS = 900;
+// Quads are used from this many projection blocks in a launch, each counted by
+// the part of its places that hold slices.  A quad gives the device an eighth of
+// the projection blocks and of the backprojection threads of its four slices, so
+// small launches lose more to latency than they save in work, and empty places
+// are work for nothing.  Quads against single slices, us per subset: 4 x 512^2,
+// 120 angles (480 blocks) 97 / 103; 12 x 256^2, 90 (540) 73 / 70; 4 x 768^2, 90
+// (540) 156 / 160; 6 x 512^2, 90 (540 of 720) 122 / 114; 3 x 1536^2, 60 (540 of
+// 720) 318 / 303; 6 x 1024^2, 45 (552 of 736) 215 / 208; 8 x 512^2, 72 (576) 97 /
+// 114; 4 x 1024^2, 80 (640) 178 / 222; 32 x 128^2, 90 (720) 55 / 58; 3 x 1024^2,
+// 120 (720 of 960) 224 / 253; 3 x 2048^2, 80 (960 of 1280) 634 / 643.
+constexpr long long QUAD_MIN_BLOCKS = 560;
+// The same for the alignment forward with its derivative, whose quads take longer:
+// 4 x 128^2, 900 angles (900) 81 / 96; 4 x 512^2, 225 (904) 163 / 184; 4 x 1024^2,
+// 113 (912) 311 / 307; 3 x 742^2, 230 (690 of 920) 203 / 202.
+constexpr long long ALIGN_QUAD_MIN_BLOCKS = 800;
 
-bool quads_fill(long long fp_block_count) { return fp_block_count >= QUAD_MIN_BLOCKS; }
+// blocks: projection blocks times the slices their quads hold, summed
+bool quads_fill(long long blocks, long long least = QUAD_MIN_BLOCKS) { return blocks >= QZ * least; }
 
 // Layers of nz equal ones that a projection of na angles takes as quads.
-int launch_quads(int nz, int px, int na)
+int launch_quads(int nz, int px, int na, long long least = QUAD_MIN_BLOCKS)
 {
     const int nq = quad_part(nz);
-    return quads_fill((long long)((nq + QZ - 1) / QZ) * fp_quad_blocks(px, na)) ? nq : 0;
+    return quads_fill((long long)nq * fp_quad_blocks(px, na), least) ? nq : 0;
 }
 
 // Layers of a uniform stack of nz that the subset drivers run as quads.
@@ -1923,7 +1930,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
                 int e = r;
                 while (e < count && slices[order[e]].n == n) ++e;
                 const int nq = tuned(c, n).fp_rays == 0 ? quad_part(e - r) : 0;
-                if (pass == 0) qblocks += (long long)((nq + QZ - 1) / QZ) * fp_quad_blocks(n, na);
+                if (pass == 0) qblocks += (long long)nq * fp_quad_blocks(n, na);
                 if (use)
                     for (int k = 0; k < nq; k += QZ) items.push_back({r + k, std::min(QZ, nq - k), 1});
                 for (int k = use ? nq : 0; k < e - r; ++k) items.push_back({r + k, 1, 0});
@@ -2266,7 +2273,7 @@ ctr_status align_forward(ctr_ctx *c, const float *img, const float *shifts, floa
     StackBind b;
     b.src = img;
     std::vector<SliceSet *> sets;
-    const int nq = std::max(g.nx, g.ny) <= LDS_FP_MAX_SIDE ? launch_quads(dN, g.px, g.pa) : 0;
+    const int nq = std::max(g.nx, g.ny) <= LDS_FP_MAX_SIDE ? launch_quads(dN, g.px, g.pa, ALIGN_QUAD_MIN_BLOCKS) : 0;
     TRY(split_stack(c, dN, nq, false, b, sets));
     for (SliceSet *S : sets) {
         TRY(run_kind(c, *S, G_PAD));
