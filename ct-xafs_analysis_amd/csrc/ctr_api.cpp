@@ -457,28 +457,51 @@ void plan_maps(SliceSet &S)
         cnt[s] = S.quad ? fp_quad_blocks(d.px, S.na) : fp_blocks(d.px, S.na, S.fp_wpb, S.fp_rays);
         const SliceDev &pd = S.h[s ? like[s - 1] : 0];
         like[s] = s > 0 && pd.nx == d.nx && pd.ny == d.ny && pd.px == d.px ? like[s - 1] : s;
-        if (S.quad && like[s] == s) {
-            const int nchunk = std::max(1, fp_blocks(d.px, 1, 4, 0));
-            for (int k = 0; k < nchunk; ++k) cost[s].push_back(mean_chord(d, (k + 0.5) * 64.0 - 0.5 * d.px) + BLOCK_COST_SAMPLES);
-        }
+        if (like[s] != s) continue;
+        // a direct-gather launch (fp_rays > 0) runs its blocks as they are numbered
+        const int nchunk = S.quad || S.fp_rays == 0 ? std::max(1, fp_blocks(d.px, 1, 4, 0)) : 1;
+        for (int k = 0; k < nchunk; ++k)
+            cost[s].push_back((S.quad ? mean_chord(d, (k + 0.5) * 64.0 - 0.5 * d.px) : (double)std::max(d.nx, d.ny)) + BLOCK_COST_SAMPLES);
     }
-    auto weight = [&](int s, int b) {       // a quad's blocks are numbered chunk by chunk
+    // Calls f(block, its weight) in launch order.  Blocks are numbered ray chunk by
+    // ray chunk, angles (of a quad: groups of them) within.  They run by families:
+    // a quarter of the angles, in parts of at most FAMILY_BLOCKS blocks, over all
+    // chunks.  Over a half turn a quarter reads one of the two image copies and
+    // walks it in one direction, so the blocks that run together on an XCD move
+    // through the same rows of it and find each other's texels in L2.  128 x
+    // 1024^2, 120 angles: 4.34 ms a launch chunk by chunk, 4.21 by quarters (240
+    // blocks each), 4.28 by eighths; 8 x 2048^2, 80 angles: 1.05, 0.94 (320), 0.86.
+    // Single slices go chunk by chunk where both copies of a slice fit in L2 or the
+    // launch is resident at once: one 2048^2, 80 angles, 176 us chunk by chunk and
+    // 164 by families, two 1024^2, 45 (1440 blocks) 61.1 and 58.6; but one 1024^2 (720
+    // blocks) 35.5 and 38.1, six 512^2 (2 MB a slice) 73.2 and 73.8, one 512^2 19.8
+    // and 20.7.
+    constexpr int FAMILY_BLOCKS = 256, FAMILY_LAUNCH = 1024;
+    constexpr size_t FAMILY_COPY_BYTES = 4u << 20;
+    long long blocks = 0;
+    for (int s = 0; s < n; ++s) blocks += cnt[s];
+    auto in_order = [&](int s, auto &&f) {
         const std::vector<double> &c = cost[like[s]];
-        if (!S.quad) return (double)std::max(S.h[s].nx, S.h[s].ny) + BLOCK_COST_SAMPLES;
-        return c[std::min(c.size() - 1, (size_t)b * c.size() / cnt[s])];
+        const int nchunk = (int)c.size();
+        const SliceDev &d = S.h[s];
+        const bool families = S.quad || (blocks > FAMILY_LAUNCH && sizeof(float) * (d.ny + 2 * PAD) * d.ipitch > FAMILY_COPY_BYTES);
+        const int ngroup = cnt[s] / nchunk;
+        const int nfam = families ? 4 * std::max(1, (nchunk * ngroup / 4 + FAMILY_BLOCKS - 1) / FAMILY_BLOCKS) : 1;
+        for (int q = 0; q < nfam; ++q)
+            for (int k = 0; k < nchunk; ++k)
+                for (int g = (int)((long long)q * ngroup / nfam); g < (int)((long long)(q + 1) * ngroup / nfam); ++g)
+                    f(k * ngroup + g, c[k]);
     };
-    for (int s = 0; s < n; ++s)
-        for (int b = 0; b < cnt[s]; ++b) total += weight(s, b);
+    for (int s = 0; s < n; ++s) in_order(s, [&](int, double w) { total += w; });
     std::vector<std::vector<std::pair<int, int>>> seg(8);
     double acc = 0.0;
     int x = 0;
     for (int s = 0; s < n; ++s)
-        for (int b = 0; b < cnt[s]; ++b) {
-            const double w = weight(s, b);
+        in_order(s, [&](int b, double w) {
             while (x < 7 && acc + 0.5 * w > total * (x + 1) / 8.0) ++x;
             seg[x].push_back({s, b});
             acc += w;
-        }
+        });
     size_t per = 0;
     for (const auto &v : seg) per = std::max(per, v.size());
     std::vector<int> &fm = S.hmap[G_FP];
