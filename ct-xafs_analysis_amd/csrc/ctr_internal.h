@@ -169,7 +169,7 @@ void launch_align_quad(const float *img, const float *imgT, size_t ifl, size_t t
 // the rows, and that copy's size in floats (slice-fastest, in chunks of 1, 4
 // or 16 slices).
 constexpr int AD_PAD = 2;
-size_t align_adj_floats(int nz, int pa, int px);
+size_t align_adj_floats(int nz, int nx, int ny, int pa, int px);
 void launch_align_adjoint(const float *prj, float *gpad, const float2 *cs, const float *shifts, float center,
                           float *img, int nz, int nx, int ny, int pa, int px, hipStream_t stream);
 void launch_align_grad(const float *pimg, const float *pimgT, int ipitch, int tpitch, const float2 *cs,

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
     (33, 47, 80, 64, 1),                        # odd D, a tall image: every column inside
     (130, 20, 150, 17, 3),                      # a wide image
     (49, 49, 40, 9, 5),                         # a detector narrower than the image
-    (64, 64, 96, 16, 17),                       # a chunk of sixteen slices and one of one
+    (64, 64, 96, 16, 17),                       # fives of four slices, the last with one
+    (272, 260, 40, 17, 17),                     # a chunk of sixteen slices and one of one
 ])
 def test_adjoint_windows(ctx, nx, ny, px, pa, dn):
     rng = np.random.default_rng(nx + 3 * ny + dn)
