@@ -180,7 +180,16 @@ struct BatchPlan {
 // code never uses its name as an address: the device address of each copy is
 // resolved once per device (hipGetSymbolAddress, with that device current, at
 // the first ctr_create on it) and kept in scratch_ptr.
-static __device__ __align__(256) char scratch[CTR_NOALLOC_SCRATCH_BYTES];
+//
+// A call's layers are held to CTR_NOALLOC_SCRATCH_BYTES with each layer's
+// descriptor counted at NOALLOC_DESC_BYTES and its backprojection map at 4 blocks
+// per compute unit, whatever the descriptor's fields for quads and the rule of
+// fill_rows make of them, so that the stacks it takes stay the same; the array has
+// NOALLOC_SLACK more for the difference (a layer takes over 330 KB, so there are
+// at most 203).
+constexpr size_t NOALLOC_DESC_BYTES = 112, NOALLOC_SLACK = 64u << 10;
+static_assert((sizeof(SliceDev) - NOALLOC_DESC_BYTES) * 204 + 8 * 256 <= NOALLOC_SLACK, "the difference fits");
+static __device__ __align__(256) char scratch[CTR_NOALLOC_SCRATCH_BYTES + NOALLOC_SLACK];
 
 constexpr int MAX_DEVICES = 64;
 std::mutex scratch_mu;
@@ -635,10 +644,9 @@ void fill_stack(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b);
 // at 4 and 25.3 at 2, six 512^2 (768 at 8) 33.1 at 8 and 31.8 at 4.  Every row
 // count gives each pixel the same sum in the same order, so only the launch shape
 // changes.
-int fill_rows(const ctr_ctx *c, const SliceSet &S, int rows)
+int fill_rows(const ctr_ctx *c, const SliceSet &S, int rows, long long want)
 {
     if (!c->adaptive_rows) return rows;
-    const long long want = 7LL * c->cus / 2;
     auto blocks = [&](int r) {
         long long n = 0;
         for (const SliceDev &d : S.h) n += bp_blocks(d.nx, d.ny, r);
@@ -683,7 +691,7 @@ void fill_stack(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b)
         d.nz = 1;
     }
     S.quad = false;
-    S.bp_rows = fill_rows(c, S, t.bp_rows);
+    S.bp_rows = fill_rows(c, S, t.bp_rows, 7LL * c->cus / 2);
 }
 
 // The descriptors of the first nz layers of a stack as quads (host only).
@@ -1191,10 +1199,16 @@ extern "C" ctr_status ctr_osem_execution_noalloc(ctr_ctx *c, float *img, float *
     StackBind none;
     fill_stack(c, S, dN, none);
     const size_t desc = (set_bytes(S) + 255) & ~(size_t)255;
-    if (desc > CTR_NOALLOC_SCRATCH_BYTES || (size_t)dN > (CTR_NOALLOC_SCRATCH_BYTES - desc) / per_layer)
+    Part parts[7];
+    set_parts(S, parts);
+    parts[0].bytes = NOALLOC_DESC_BYTES * (size_t)dN;
+    const int rows4 = fill_rows(c, S, tuned(c, std::max(g.nx, g.ny)).bp_rows, 4LL * c->cus);
+    parts[1 + G_BP].bytes = sizeof(int) * (size_t)dN * bp_blocks(g.nx, g.ny, rows4);
+    const size_t counted = (parts_bytes(parts, 7) + 255) & ~(size_t)255;
+    if (counted > CTR_NOALLOC_SCRATCH_BYTES || (size_t)dN > (CTR_NOALLOC_SCRATCH_BYTES - counted) / per_layer)
         return fail(c, CTR_INVALID_ARGUMENT,
                     "%d layers of %d x %d with %d bins need %zu bytes of scratch; the no-allocation driver has %zu",
-                    dN, g.nx, g.ny, g.px, desc + (size_t)dN * per_layer, (size_t)CTR_NOALLOC_SCRATCH_BYTES);
+                    dN, g.nx, g.ny, g.px, counted + (size_t)dN * per_layer, (size_t)CTR_NOALLOC_SCRATCH_BYTES);
     HIPTRY(c, hipSetDevice(c->device));
     char *base = c->scratch + desc;
     StackBind b;
@@ -2017,7 +2031,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
             orr += (size_t)(m.quad ? QZ : 1) * na * l.rpitch;
         }
         for (auto &S : P.sets) {
-            if (!S->quad) S->bp_rows = fill_rows(c, *S, S->bp_rows);
+            if (!S->quad) S->bp_rows = fill_rows(c, *S, S->bp_rows, 7LL * c->cus / 2);
             TRY(upload_set(c, *S));
         }
     }
