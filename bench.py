@@ -87,18 +87,18 @@ def no_gc():
 METRIC = "batched OS-EM slice-iters/s vs per-slice launch, 1024² 1200 proj, relerr≤1e-4"
 PEAK_FP32_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
-# LDS read rate of the device: conflict-free ds_read2_b32, 275 bytes per ns
-# per CU measured on MI355X (128 bytes per clock), over its 256 CUs.  The
-# projector reads 16 bytes of LDS per bilinear sample (two ds_read2_b32 of
-# two texels each).
-LDS_READ_TBS = 275.0 * 256 / 1e3
+# LDS read rate of the device: conflict-free ds_read_b128, 412 bytes per ns
+# per CU measured on MI355X, over its 256 CUs (ds_read2_b32: 240 to 275).  The
+# projector reads 16 bytes of LDS per bilinear sample of a slice (a quad's four
+# slices: four ds_read_b128).
+LDS_READ_TBS = 412.0 * 256 / 1e3
 FP_LDS_BYTES_PER_SAMPLE = 16.0
 # Bytes moved past L2 per forward-projection launch, per slice of 1024^2 with
 # 120 angles (one subset of 1200): rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE on
-# the 128-slice k_fp_lds<0> launch, scaled by the same counters on a plain
+# the 128-slice k_fp_quad<0> launch, scaled by the same counters on a plain
 # 256 MiB copy (FETCH x 1.99969, WRITE x 1.0), divided by 128
-# (profiles/k_fp_lds_k_bp_osem_1024sq_1200proj_128slices.md).
-FP_TRAFFIC_BYTES_PER_SLICE = 44102141.0
+# (profiles/k_fp_quad_k_bp_quad_osem_1024sq_1200proj_128slices.md).
+FP_TRAFFIC_BYTES_PER_SLICE = 79104960.0
 FP_TRAFFIC_SHAPE = (1024, 1200, 10)
 # Bytes moved past L2 per k_reslice launch for 1600 projections of 2048 x 2048
 # (rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE scaled the same way; the 9 rows a
@@ -670,7 +670,8 @@ def main():
     log(f"per-slice launch: {per_slice:.2f} (1024^2-equivalent) slice-iters/s")
 
     kinds = sorted({(tune[m]["fp_rays"], tune[m]["fp_tile"]) for m in set(sides)} if tune else {(0, 60)})
-    fp_kernel = " + ".join(f"k_fp_lds<FP_RATIO, {tile}>" if rays == 0 else "k_fp<FP_RATIO>" for rays, tile in kinds)
+    fp_kernel = " + ".join(f"k_fp_quad<FP_RATIO> (slices not in quads: k_fp_lds<FP_RATIO, {tile}>)" if rays == 0
+                           else "k_fp<FP_RATIO>" for rays, tile in kinds)
     fp_tile60 = kinds == [(0, 60)]
     fp_flops = sum(14.0 * m * na * m for m in sides)          # 14 FLOP per bilinear sample, D = m samples per ray
     fp_bytes = sum(4 * m * m + 8 * na * m for m in sides)    # image once, measured rows in, ratio rows out
