@@ -746,22 +746,41 @@ constexpr long long QUAD_MIN_BLOCKS = 560;
 // 113 (912) 311 / 307; 3 x 742^2, 230 (690 of 920) 203 / 202.
 constexpr long long ALIGN_QUAD_MIN_BLOCKS = 800;
 
+// A quad's backprojection sums all angles of 64 x 16 pixels in one block, so small
+// images with many angles need this many of them: 32 x 128^2, 90 angles (128) 55
+// us a subset and 58 as single slices; 8 x 131^2, 261 angles (54) 100 and 76.
+constexpr long long QUAD_MIN_BP_BLOCKS = 112;
+// The two angles of a quad's projection block share a window while the rims of
+// their strips lie close: 21 x 1221^2, 23 angles (83 texels) take 1.25 times the
+// single slices' time, 4 x 2048^2, 40 angles (80) 0.96, 4 x 1536^2, 60 angles (40)
+// 0.86, 4 x 1024^2, 80 angles (20) 0.80.
+constexpr double QUAD_MAX_RIM_TEXELS = 56.0;
+
 // blocks: projection blocks times the slices their quads hold, summed
 bool quads_fill(long long blocks, long long least = QUAD_MIN_BLOCKS) { return blocks >= QZ * least; }
 
-// Layers of nz equal ones that a projection of na angles takes as quads.
-int launch_quads(int nz, int px, int na, long long least = QUAD_MIN_BLOCKS)
+// How far apart the rims of strips at neighbouring angles of a subset lie on
+// average, in texels of a side D (angles `stride` apart in the table).
+double rim_texels(const ctr_ctx *c, int D, int stride)
 {
-    const int nq = quad_part(nz);
-    return quads_fill((long long)nq * fp_quad_blocks(px, na), least) ? nq : 0;
+    const int n = (int)c->ang.size();
+    double sum = 0.0;
+    int k = 0;
+    for (int a = 0; a + stride < n; a += stride, ++k) {
+        const double step = std::fabs(std::remainder((double)c->ang[a + stride] - (double)c->ang[a], 180.0));
+        sum += step * (M_PI / 180.0);
+    }
+    return k > 0 ? sum / k * 0.5 * D : 0.0;
 }
 
 // Layers of a uniform stack of nz that the subset drivers run as quads.
 int stack_quads(ctr_ctx *c, int nz)
 {
     const ctr_geometry &g = c->g;
-    if (tuned(c, std::max(g.nx, g.ny)).fp_rays != 0) return 0;
-    return launch_quads(nz, g.px, g.pa / g.ss);
+    const int D = std::max(g.nx, g.ny), nq = quad_part(nz);
+    if (tuned(c, D).fp_rays != 0 || !quads_fill((long long)nq * fp_quad_blocks(g.px, g.pa / g.ss))) return 0;
+    const long long bp = (long long)((nq + QZ - 1) / QZ) * bp_blocks(g.nx, g.ny, QBP_ROWS);
+    return bp >= QUAD_MIN_BP_BLOCKS && rim_texels(c, D, g.ss) <= QUAD_MAX_RIM_TEXELS ? nq : 0;
 }
 
 // Device workspace for an nz-layer stack of the current geometry.
@@ -1958,16 +1977,19 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
             int at, n, quad;                   // first place in `order`, slices, held as one quad
         };
         std::vector<Item> items;
-        long long qblocks = 0;
+        long long qblocks = 0, qbp = 0;
         for (int pass = 0; pass < 2; ++pass) {
-            const bool use = pass == 1 && quads_fill(qblocks);
+            const bool use = pass == 1 && quads_fill(qblocks) && qbp >= QUAD_MIN_BP_BLOCKS;
             items.clear();
             for (int r = 0; r < count;) {
                 const int n = slices[order[r]].n;
                 int e = r;
                 while (e < count && slices[order[e]].n == n) ++e;
-                const int nq = tuned(c, n).fp_rays == 0 ? quad_part(e - r) : 0;
-                if (pass == 0) qblocks += (long long)nq * fp_quad_blocks(n, na);
+                const int nq = tuned(c, n).fp_rays == 0 && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS ? quad_part(e - r) : 0;
+                if (pass == 0) {
+                    qblocks += (long long)nq * fp_quad_blocks(n, na);
+                    qbp += (long long)((nq + QZ - 1) / QZ) * bp_blocks(n, n, QBP_ROWS);
+                }
                 if (use)
                     for (int k = 0; k < nq; k += QZ) items.push_back({r + k, std::min(QZ, nq - k), 1});
                 for (int k = use ? nq : 0; k < e - r; ++k) items.push_back({r + k, 1, 0});
@@ -2310,7 +2332,10 @@ ctr_status align_forward(ctr_ctx *c, const float *img, const float *shifts, floa
     StackBind b;
     b.src = img;
     std::vector<SliceSet *> sets;
-    const int nq = std::max(g.nx, g.ny) <= LDS_FP_MAX_SIDE ? launch_quads(dN, g.px, g.pa, ALIGN_QUAD_MIN_BLOCKS) : 0;
+    const int D = std::max(g.nx, g.ny), part = quad_part(dN);
+    const bool quads = D <= LDS_FP_MAX_SIDE && quads_fill((long long)part * fp_quad_blocks(g.px, g.pa), ALIGN_QUAD_MIN_BLOCKS) &&
+                       rim_texels(c, D, 1) <= QUAD_MAX_RIM_TEXELS;
+    const int nq = quads ? part : 0;
     TRY(split_stack(c, dN, nq, false, b, sets));
     for (SliceSet *S : sets) {
         TRY(run_kind(c, *S, G_PAD));

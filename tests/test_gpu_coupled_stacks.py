@@ -14,10 +14,10 @@ from _util import dev, host, say
 pytestmark = pytest.mark.gpu
 
 CASES = [
-    # nx, ny, px, pa, ss, dn: at least 900 projection blocks run as quads
-    (66, 53, 130, 1200, 2, 6),                  # a quad and a quad with two
-    (64, 64, 64, 1800, 2, 9),                   # whole tiles; one slice left over
-    (127, 35, 65, 1802, 2, 7),                  # one column short, three rows over, a quad with three
+    # nx, ny, px, pa, ss, dn: at least 560 filled projection and 112 backprojection blocks run as quads
+    (66, 53, 130, 130, 2, 58),                  # whole quads and one with two
+    (64, 64, 64, 180, 2, 113),                  # whole tiles; one slice left over
+    (127, 35, 65, 182, 2, 79),                  # one column short, three rows over, a quad with three
     (33, 130, 97, 90, 3, 5),                    # single slices only
     (65, 17, 40, 60, 4, 1),                     # one slice: it is its own layer neighbour
 ]

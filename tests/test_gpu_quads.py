@@ -30,7 +30,7 @@ def _angles(kind, pa, rng):
     (127, 127, 127, 240, 2, 35, "random"),      # a quad with three slices
     (150, 97, 170, 105, 1, 34, "wide"),         # rectangular, wide detector, a quad with two
     (97, 150, 61, 300, 1, 33, "dense"),         # narrow detector, one slice left over
-    (20, 20, 20, 512, 1, 16, "random"),         # smaller than a chunk and a block
+    (20, 20, 20, 64, 1, 226, "random"),         # smaller than a chunk and a block
     (512, 512, 512, 90, 1, 12, "wide"),
     (1024, 1024, 1024, 240, 2, 4, "dense"),
 ])
