@@ -741,6 +741,12 @@ int quad_part(int n) { return n >= QZ - 1 && n % QZ >= 2 ? n : n / QZ * QZ; }
 // 114; 4 x 1024^2, 80 (640) 178 / 222; 32 x 128^2, 90 (720) 55 / 58; 3 x 1024^2,
 // 120 (720 of 960) 224 / 253; 3 x 2048^2, 80 (960 of 1280) 634 / 643.
 constexpr long long QUAD_MIN_BLOCKS = 560;
+// The same for an uneven batch that also leaves single slices, whose launches come
+// on top: 41 slices of 189^2 to 511^2, 42 angles (929 blocks) 1.21 ms a call with
+// quads and 1.02 all single; 30 of 185^2 to 1109^2, 62 angles (1270) 24.0 and 21.8;
+// 59 of 255^2 to 1024^2, 120 angles (over 5000) 11.9, and 20.1 with the single
+// slices' kernels of before.
+constexpr long long QUAD_MIN_BLOCKS_BESIDE_SINGLES = 1800;
 // The same for the alignment forward with its derivative, whose quads take longer:
 // 4 x 128^2, 900 angles (900) 81 / 96; 4 x 512^2, 225 (904) 163 / 184; 4 x 1024^2,
 // 113 (912) 311 / 307; 3 x 742^2, 230 (690 of 920) 203 / 202.
@@ -1977,9 +1983,10 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
             int at, n, quad;                   // first place in `order`, slices, held as one quad
         };
         std::vector<Item> items;
-        long long qblocks = 0, qbp = 0;
+        long long qblocks = 0, qbp = 0, left = 0;
         for (int pass = 0; pass < 2; ++pass) {
-            const bool use = pass == 1 && quads_fill(qblocks) && qbp >= QUAD_MIN_BP_BLOCKS;
+            const bool use = pass == 1 && qbp >= QUAD_MIN_BP_BLOCKS &&
+                             quads_fill(qblocks, left > 0 ? QUAD_MIN_BLOCKS_BESIDE_SINGLES : QUAD_MIN_BLOCKS);
             items.clear();
             for (int r = 0; r < count;) {
                 const int n = slices[order[r]].n;
@@ -1987,6 +1994,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
                 while (e < count && slices[order[e]].n == n) ++e;
                 const int nq = tuned(c, n).fp_rays == 0 && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS ? quad_part(e - r) : 0;
                 if (pass == 0) {
+                    left += e - r - nq;
                     qblocks += (long long)nq * fp_quad_blocks(n, na);
                     qbp += (long long)((nq + QZ - 1) / QZ) * bp_blocks(n, n, QBP_ROWS);
                 }
