@@ -263,6 +263,7 @@ ctr_status fail(ctr_ctx *c, ctr_status st, const char *fmt, ...)
 
 ctr_status hipfail(ctr_ctx *c, const char *what, hipError_t e)
 {
+    (void)hipGetLastError();                 // reported here: the next call's checks start clean
     return fail(c, e == hipErrorOutOfMemory ? CTR_OUT_OF_MEMORY : CTR_HIP_ERROR, "%s: %s", what,
                 hipGetErrorString(e));
 }
@@ -1968,8 +1969,10 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
     const int na = c->g.pa / c->g.ss;
     if (!c->plan || !same_key(c->plan->key, slices, count)) {
         HIPTRY(c, hipStreamSynchronize(c->stream));
-        c->plan.reset(new BatchPlan());
-        BatchPlan &P = *c->plan;
+        c->plan.reset();
+        // the context takes the plan once it is whole: a build that fails leaves none
+        auto built = std::make_unique<BatchPlan>();
+        BatchPlan &P = *built;
         P.key.assign(slices, slices + count);
         // largest slices first: their blocks start earliest, evening out the tail
         std::vector<int> order(count);
@@ -2064,6 +2067,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
             if (!S->quad) S->bp_rows = fill_rows(c, *S, S->bp_rows, 7LL * c->cus / 2);
             TRY(upload_set(c, *S));
         }
+        c->plan = std::move(built);
     }
     BatchPlan &P = *c->plan;
     for (auto &S : P.sets) {
