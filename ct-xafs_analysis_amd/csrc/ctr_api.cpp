@@ -1194,11 +1194,12 @@ extern "C" ctr_status ctr_osem_execution(ctr_ctx *c, float *img, float *prj, int
     TRY(require_full_grid(c));
     const ctr_geometry &g = c->g;
     HIPTRY(c, hipSetDevice(c->device));
-    if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     StackBind b;
     b.prj = prj; b.src = img; b.dst = img;
     std::vector<SliceSet *> sets;
     TRY(split_stack(c, dN, stack_quads(c, dN), true, b, sets));
+    // only now, when nothing more is allocated: a call that fails has not corrected
+    if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     // the layers are independent: each part runs all its iterations
     for (SliceSet *S : sets) TRY(osem_iterations(c, *S, it));
     return CTR_OK;
@@ -1295,11 +1296,11 @@ extern "C" ctr_status ctr_fista_osem_execution(ctr_ctx *c, float *img, float *pr
     HIPTRY(c, c->w_l2.ensure(sizeof(float) * g.ss));
     launch_fill(c->w_l2.f(), g.ss, 0.5f, c->stream);
     POST(c, "fill L2norm");
-    if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     StackBind b;
     b.prj = prj; b.src = img; b.dst = img; b.aux = c->w_aux1.f();
     std::vector<SliceSet *> sets;
     TRY(split_stack(c, dN, stack_quads(c, dN), true, b, sets));
+    if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     for (SliceSet *S : sets) {
         TRY(run_kind(c, *S, G_PAD));
         TRY(run_kind(c, *S, G_TR));
@@ -1329,12 +1330,12 @@ extern "C" ctr_status ctr_aart_execution(ctr_ctx *c, float *img, float *prj, int
     TRY(require_full_grid(c));
     const ctr_geometry &g = c->g;
     HIPTRY(c, hipSetDevice(c->device));
-    if (g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     const float alpha = (g.mode == 3) ? g.wt2 : g.wt1;   // GPU.cpp:1161-1165
     StackBind b;
     b.prj = prj; b.src = img; b.dst = img;
     std::vector<SliceSet *> sets;
     TRY(split_stack(c, dN, stack_quads(c, dN), true, b, sets));
+    if (g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     for (SliceSet *S : sets) {
         // zero borders of both copies (the interior is overwritten next)
         TRY(run_kind(c, *S, G_PAD));

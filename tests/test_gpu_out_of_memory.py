@@ -1,7 +1,10 @@
 """Calls whose workspace does not fit the device: they report out of memory, again
-when called again, and the next call that fits runs.  The stacks are nominally large (sides of 16384, a detector of a few bins)
+when called again, leave the caller's buffers as they were, and the next call that
+fits runs.  The stacks are nominally large (sides of 16384, a detector of a few bins)
 so that the first allocation that fails is far beyond any device's memory; nothing
 runs on the images, which are small buffers here."""
+import ctypes as C
+
 import numpy as np
 import pytest
 from ctrecon import Context
@@ -46,4 +49,20 @@ def test_batched_list_too_large(own):
     own.osem_batched(imgs, prjs, 1, use_graph=True)
     own.synchronize()
     assert not (host(imgs[0]) == 1.0).all()
+    _small_run(own)
+
+
+@pytest.mark.parametrize("driver", ["ctr_osem_execution", "ctr_fista_osem_execution", "ctr_aart_execution"])
+def test_stack_too_large_keeps_its_sinograms(own, driver):
+    pa, ss, px = 4, 2, 8
+    own.set_geometry(SIDE, px, pa, ss, mode=2, correction_mode=1, angles_deg=np.arange(pa, dtype=np.float32) * 45.0)
+    x, y0 = dev(np.ones((64, 64))), np.random.default_rng(2).uniform(1.0, 9.0, (COUNT, pa, px)).astype(np.float32)
+    y = dev(y0)
+    say("stack too large", driver)
+    args = [own.h, C.c_void_p(x.data_ptr()), C.c_void_p(y.data_ptr()), COUNT, 1] + ([1] if driver != "ctr_aart_execution" else [])
+    for _ in range(2):
+        st = getattr(own.lib, driver)(*args)
+        assert st == CTR_OUT_OF_MEMORY, own.lib.ctr_last_error(own.h)
+        own.synchronize()
+        assert np.array_equal(host(y), y0)
     _small_run(own)
