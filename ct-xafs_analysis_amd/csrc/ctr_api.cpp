@@ -331,7 +331,8 @@ size_t parts_bytes(const Part *parts, int n)
 ctr_status stage_upload(ctr_ctx *c, void *dst, const Part *parts, int n, bool may_grow)
 {
     Staging &st = c->stage;
-    const size_t total = std::max(parts_bytes(parts, n), (size_t)16);
+    const size_t total = parts_bytes(parts, n);
+    if (total == 0) return CTR_OK;
     if (total > st.cap) {
         if (!may_grow)
             return fail(c, CTR_INVALID_ARGUMENT, "upload of %zu bytes exceeds the %zu-byte staging ring", total,
