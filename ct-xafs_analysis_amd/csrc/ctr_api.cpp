@@ -150,6 +150,7 @@ size_t pimgT_floats(const Layout &l) { return (size_t)(l.nx + 2 * PAD) * l.tpitc
 // per wave and fp_wpb waves per block; bp_rows rows per backprojection thread.
 struct Tune {
     int fp_wpb = 4, fp_rays = 0, fp_tile = 60, bp_rows = 8;   // the defaults
+    bool asked = false;      // the caller set it, other than the defaults: the side runs as it says
     bool operator==(const Tune &o) const
     {
         return fp_wpb == o.fp_wpb && fp_rays == o.fp_rays && fp_tile == o.fp_tile && bp_rows == o.bp_rows;
@@ -727,6 +728,15 @@ void fill_quads(ctr_ctx *c, SliceSet &S, int nz, const StackBind &b)
     }
 }
 
+// Whether slices of side n may run as quads, which have a shape of their own: not
+// where the caller set a schedule for the side or asked for its rows as set.  The
+// tuner's pick is no such wish: it times single slices only.
+bool quads_allowed(ctr_ctx *c, int n)
+{
+    auto it = c->tune.find(n);
+    return n <= LDS_FP_MAX_SIDE && c->adaptive_rows && !(it != c->tune.end() && it->second.asked);
+}
+
 // How many of n equal slices run as quads: all whole quads, and two or three
 // left over as a quad with empty places (a quad takes about two slices' time,
 // so a lone pair stays single).
@@ -786,7 +796,7 @@ int stack_quads(ctr_ctx *c, int nz)
 {
     const ctr_geometry &g = c->g;
     const int D = std::max(g.nx, g.ny), nq = quad_part(nz);
-    if (tuned(c, D).fp_rays != 0 || !quads_fill((long long)nq * fp_quad_blocks(g.px, g.pa / g.ss))) return 0;
+    if (!quads_allowed(c, D) || !quads_fill((long long)nq * fp_quad_blocks(g.px, g.pa / g.ss))) return 0;
     const long long bp = (long long)((nq + QZ - 1) / QZ) * bp_blocks(g.nx, g.ny, QBP_ROWS);
     return bp >= QUAD_MIN_BP_BLOCKS && rim_texels(c, D, g.ss) <= QUAD_MAX_RIM_TEXELS ? nq : 0;
 }
@@ -1997,7 +2007,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
                 const int n = slices[order[r]].n;
                 int e = r;
                 while (e < count && slices[order[e]].n == n) ++e;
-                const int nq = tuned(c, n).fp_rays == 0 && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS ? quad_part(e - r) : 0;
+                const int nq = quads_allowed(c, n) && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS ? quad_part(e - r) : 0;
                 if (pass == 0) {
                     left += e - r - nq;
                     qblocks += (long long)nq * fp_quad_blocks(n, na);
@@ -2157,6 +2167,7 @@ extern "C" ctr_status ctr_set_schedule(ctr_ctx *c, int n, const ctr_schedule *s)
     t.fp_wpb = s->fp_waves;
     t.fp_tile = s->fp_rays == 0 ? s->fp_tile : 60;
     t.bp_rows = s->bp_rows;
+    t.asked = !(t == Tune{});
     c->tune[n] = t;
     if (c->plan) {
         // the cached batched plan holds the old schedule: rebuild it, once

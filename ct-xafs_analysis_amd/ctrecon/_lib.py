@@ -592,9 +592,10 @@ class Context:
         return {k: d[k] for k in ("fp_rays", "fp_waves", "fp_tile", "bp_rows")}
 
     def set_adaptive_rows(self, on):
-        """on (the default): stacks too small to give the device 4
+        """on (the default): stacks too small to give the device 3.5
         backprojection blocks per compute unit run with fewer rows per thread
-        than their side's schedule; off: every stack runs its schedule as set.
+        than their side's schedule; off: every stack runs its schedule as set,
+        slice by slice (none four side by side).
         The images are the same either way."""
         self._run(self.lib.ctr_set_adaptive_rows, (self.h, int(bool(on)),), "ctr_set_adaptive_rows")
 

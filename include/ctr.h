@@ -337,9 +337,12 @@ ctr_status ctr_tv_prox_2d(ctr_ctx *ctx, const float *v, float *x_new, int dN, fl
 ctr_status ctr_osem_batched(ctr_ctx *ctx, const ctr_slice *slices, int count, int it,
                             int use_graph);
 
-/* A projector / backprojector schedule for one slice side.  No reference
- * counterpart: the reference fixes its work-group shape per compiled program
- * (GPU.cpp:169-172, 538-547). */
+/* A projector / backprojector schedule for one slice side.  It applies to
+ * slices that run one by one; where a side has enough of them, OS-EM, TV OS-EM,
+ * AART and batched stacks run four slices side by side with a shape of their
+ * own (the same images bit for bit as under the LDS-tiled schedules).  No
+ * reference counterpart: the reference fixes its work-group shape per compiled
+ * program (GPU.cpp:169-172, 538-547). */
 typedef struct ctr_schedule {
     int fp_rays;    /* 0: the LDS-tiled projector; 64 / 32 / 16 / 8: the direct-gather one, rays per wave */
     int fp_waves;   /* waves per projection block: 4 for the LDS-tiled projector, 2 or 4 otherwise */
@@ -352,18 +355,22 @@ typedef struct ctr_schedule {
 
 /* Times the projector schedules (LDS tiles of 60 / 44 / 32 samples, direct
  * gathers of 64 / 32 / 16 / 8 rays per wave with 2 or 4 waves per block) and
- * the backprojection row counts on a batch-sized launch of side n, keeps the
- * fastest for side n and writes it (with its and the default's times) to
- * *best.  Blocks the host.  Batched stacks run each side's schedule. */
+ * the backprojection row counts on a batch-sized launch of side n, slice by
+ * slice, keeps the fastest for side n and writes it (with its and the default's
+ * times) to *best.  Blocks the host.  The pick decides how the side's single
+ * slices run, not which slices run four side by side. */
 ctr_status ctr_autotune(ctr_ctx *ctx, int n, ctr_schedule *best);
-/* Sets the schedule of side n (the time fields are ignored). */
+/* Sets the schedule of side n (the time fields are ignored).  Under any but the
+ * default schedule (tile 60, 8 rows) every slice of the side runs as it says,
+ * one by one; the default puts the side back to how it ran at first. */
 ctr_status ctr_set_schedule(ctr_ctx *ctx, int n, const ctr_schedule *schedule);
-/* The schedule side n runs (the defaults unless tuned or set). */
+/* The schedule side n's single slices run (the defaults unless tuned or set). */
 ctr_status ctr_get_schedule(ctr_ctx *ctx, int n, ctr_schedule *schedule);
 /* enable != 0 (the default): a stack whose backprojection would have fewer
- * than 4 blocks per compute unit at its side's bp_rows runs with bp_rows
+ * than 3.5 blocks per compute unit at its side's bp_rows runs with bp_rows
  * halved until it has them or reaches 1 (one 512^2 slice: 1 row, 1024
- * blocks).  0: every stack runs its side's bp_rows as set.  The images are
+ * blocks).  0: every stack runs its side's bp_rows as set, slice by slice
+ * (none four side by side).  The images are
  * the same either way (every row count sums each pixel's angles in the same
  * order); only the launch shape changes.  No reference counterpart. */
 ctr_status ctr_set_adaptive_rows(ctr_ctx *ctx, int enable);
