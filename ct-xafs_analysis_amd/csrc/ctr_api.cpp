@@ -737,8 +737,8 @@ bool quads_allowed(ctr_ctx *c, int n)
     return n <= LDS_FP_MAX_SIDE && c->adaptive_rows && !(it != c->tune.end() && it->second.asked);
 }
 
-// How many of n equal slices run as quads: all whole quads, and two or three
-// left over as a quad with empty places (a quad takes about two slices' time,
+// How many of n equal slices run as quads beside others: all whole quads, and two or
+// three left over as a quad with empty places (a quad takes about two slices' time,
 // so a lone pair stays single).
 int quad_part(int n) { return n >= QZ - 1 && n % QZ >= 2 ? n : n / QZ * QZ; }
 
@@ -746,23 +746,43 @@ int quad_part(int n) { return n >= QZ - 1 && n % QZ >= 2 ? n : n / QZ * QZ; }
 // the part of its places that hold slices.  A quad gives the device an eighth of
 // the projection blocks and of the backprojection threads of its four slices, so
 // small launches lose more to latency than they save in work, and empty places
-// are work for nothing.  Quads against single slices, us per subset: 4 x 512^2,
-// 120 angles (480 blocks) 97 / 103; 12 x 256^2, 90 (540) 73 / 70; 4 x 768^2, 90
-// (540) 156 / 160; 6 x 512^2, 90 (540 of 720) 122 / 114; 3 x 1536^2, 60 (540 of
-// 720) 318 / 303; 6 x 1024^2, 45 (552 of 736) 215 / 208; 8 x 512^2, 72 (576) 97 /
-// 114; 4 x 1024^2, 80 (640) 178 / 222; 32 x 128^2, 90 (720) 55 / 58; 3 x 1024^2,
-// 120 (720 of 960) 224 / 253; 3 x 2048^2, 80 (960 of 1280) 634 / 643.
+// are work for nothing.  Quads against single slices, us per subset of a call of
+// four: 16 x 300^2, 50 angles (500 blocks) 92 / 84; 11 x 512^2, 50 (550 of 600) 137 /
+// 131; 7 x 384^2, 110 (577 of 660) 114 / 111; 10 x 1024^2, 30 (600 of 720) 258 / 248;
+// 6 x 640^2, 80 (600 of 800) 146 / 163; 8 x 512^2, 80 (640) 114 / 139; 4 x 1024^2, 80
+// (640) 193 / 240; 12 x 256^2, 110 (660) 94 / 94; 16 x 300^2, 80 (800) 93 / 112.
 constexpr long long QUAD_MIN_BLOCKS = 560;
-// The same for an uneven batch that also leaves single slices, whose launches come
-// on top: 41 slices of 189^2 to 511^2, 42 angles (929 blocks) 1.21 ms a call with
+// One slice left over (n % 4 == 1): a launch of its own takes far longer than the
+// slice adds to a launch of all, and a quad for it alone is mostly work for nothing.
+// Up to this side, and this much work in a quad (projection blocks times side), the
+// quad is the cheaper of the two, and both need more blocks than whole quads do.  A
+// quad more / the slice singly after the others / all singly: 33 x 128^2, 160 angles
+// (1320 blocks with it) 93 / 112 / 107; 17 x 256^2, 120 (1020) 110 / 123 / 126; 9 x
+// 512^2, 90 (810) 182 / 179 / 172; 13 x 512^2, 120 (1560) 211 / 228 / 290; 9 x 640^2, 60
+// (600 without it) 184 / 198 / 177; 9 x 640^2, 90 (900) 235 / 225 / 241; 9 x 768^2, 90
+// (1080) 304 / 280 / 326; 5 x 1024^2, 90 (720) 308 / 329 / 318; 5 x 1024^2, 120 (960)
+// 365 / 334 / 398; 5 x 2048^2, 60 (960) 994 / 688 / 799.
+constexpr int QUAD_ONE_OVER_SIDE = 512;
+constexpr long long QUAD_ONE_OVER_WORK = 350000;
+constexpr long long QUAD_MIN_BLOCKS_ONE_SMALL = 900, QUAD_MIN_BLOCKS_ONE_LARGE = 640;
+// The same for batches of several sides that also leave single slices, whose launches
+// come on top: 41 slices of 189^2 to 511^2, 42 angles (929 blocks) 1.21 ms a call with
 // quads and 1.02 all single; 30 of 185^2 to 1109^2, 62 angles (1270) 24.0 and 21.8;
 // 59 of 255^2 to 1024^2, 120 angles (over 5000) 11.9, and 20.1 with the single
 // slices' kernels of before.
 constexpr long long QUAD_MIN_BLOCKS_BESIDE_SINGLES = 1800;
 // The same for the alignment forward with its derivative, whose quads take longer:
 // 4 x 128^2, 900 angles (900) 81 / 96; 4 x 512^2, 225 (904) 163 / 184; 4 x 1024^2,
-// 113 (912) 311 / 307; 3 x 742^2, 230 (690 of 920) 203 / 202.
+// 113 (912) 311 / 307; 3 x 742^2, 230 (690 of 920) 203 / 202.  With one layer left
+// over, a quad more / the layer singly after / all singly: 9 x 200^2, 200 angles (900
+// with it) 109 / 125 / 103; 13 x 128^2, 400 (1300) 94 / 123 / 108; 9 x 384^2, 200 (1350)
+// 202 / 215 / 200; 9 x 256^2, 400 (1800) 173 / 187 / 185; 9 x 256^2, 900 (4050, past the
+// work line) 308 / 294 / 340; five layers gain by no quad more: 5 x 200^2, 900 (1800
+// without it) 196 / 189 / 182; 5 x 512^2, 300 (1200) - / 261 / 259, without the
+// derivative - / 230 / 237; 5 x 512^2, 400 (1600) 340 / 297 / 325; 5 x 742^2, 200 (1200)
+// 367 / 352 / 341.
 constexpr long long ALIGN_QUAD_MIN_BLOCKS = 800;
+constexpr long long ALIGN_QUAD_MIN_BLOCKS_ONE_IN = 1200, ALIGN_QUAD_MIN_BLOCKS_ONE_BESIDE = 1200;
 
 // A quad's backprojection sums all angles of 64 x 16 pixels in one block, so small
 // images with many angles need this many of them: 32 x 128^2, 90 angles (128) 55
@@ -775,7 +795,7 @@ constexpr long long QUAD_MIN_BP_BLOCKS = 112;
 constexpr double QUAD_MAX_RIM_TEXELS = 56.0;
 
 // blocks: projection blocks times the slices their quads hold, summed
-bool quads_fill(long long blocks, long long least = QUAD_MIN_BLOCKS) { return blocks >= QZ * least; }
+bool quads_fill(long long blocks, long long least) { return blocks >= QZ * least; }
 
 // How far apart the rims of strips at neighbouring angles of a subset lie on
 // average, in texels of a side D (angles `stride` apart in the table).
@@ -791,14 +811,39 @@ double rim_texels(const ctr_ctx *c, int D, int stride)
     return k > 0 ? sum / k * 0.5 * D : 0.0;
 }
 
+// Whether one slice left over of side D joins as a quad (of per_quad projection blocks).
+bool one_joins(int D, int per_quad) { return D <= QUAD_ONE_OVER_SIDE && (long long)per_quad * D <= QUAD_ONE_OVER_WORK; }
+
+// How many of n equal slices of side D run as quads where they are all there is.
+// per_quad, bp_per_quad: a quad's projection and backprojection blocks.
+int quads_of(int n, int D, int per_quad, int bp_per_quad)
+{
+    if (n < QZ - 1) return 0;
+    const bool one = n % QZ == 1;
+    const int nq = one && !one_joins(D, per_quad) ? n - 1 : n;
+    const long long least = !one ? QUAD_MIN_BLOCKS : (D <= QUAD_ONE_OVER_SIDE ? QUAD_MIN_BLOCKS_ONE_SMALL : QUAD_MIN_BLOCKS_ONE_LARGE);
+    return quads_fill((long long)nq * per_quad, least) && (long long)((nq + QZ - 1) / QZ) * bp_per_quad >= QUAD_MIN_BP_BLOCKS
+               ? nq : 0;
+}
+
+// The same for the layers of an alignment forward.
+int align_quads_of(int n, int D, int per_quad)
+{
+    if (n < QZ - 1) return 0;
+    const bool one = n % QZ == 1, in = one && n > 2 * QZ && one_joins(D, per_quad);
+    const int nq = one && !in ? n - 1 : n;
+    const long long least = in ? ALIGN_QUAD_MIN_BLOCKS_ONE_IN : (one ? ALIGN_QUAD_MIN_BLOCKS_ONE_BESIDE : ALIGN_QUAD_MIN_BLOCKS);
+    return quads_fill((long long)nq * per_quad, least) ? nq : 0;
+}
+
 // Layers of a uniform stack of nz that the subset drivers run as quads.
 int stack_quads(ctr_ctx *c, int nz)
 {
     const ctr_geometry &g = c->g;
-    const int D = std::max(g.nx, g.ny), nq = quad_part(nz);
-    if (!quads_allowed(c, D) || !quads_fill((long long)nq * fp_quad_blocks(g.px, g.pa / g.ss))) return 0;
-    const long long bp = (long long)((nq + QZ - 1) / QZ) * bp_blocks(g.nx, g.ny, QBP_ROWS);
-    return bp >= QUAD_MIN_BP_BLOCKS && rim_texels(c, D, g.ss) <= QUAD_MAX_RIM_TEXELS ? nq : 0;
+    const int D = std::max(g.nx, g.ny);
+    if (!quads_allowed(c, D)) return 0;
+    const int nq = quads_of(nz, D, fp_quad_blocks(g.px, g.pa / g.ss), bp_blocks(g.nx, g.ny, QBP_ROWS));
+    return nq > 0 && rim_texels(c, D, g.ss) <= QUAD_MAX_RIM_TEXELS ? nq : 0;
 }
 
 // Device workspace for an nz-layer stack of the current geometry.
@@ -1991,23 +2036,27 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
         for (int i = 0; i < count; ++i) order[i] = i;
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return slices[a].n > slices[b].n; });
         // Runs of equal sides in that order: the part of a run that goes as
-        // quads, and the slices left.  One set of quads, and one set of single
+        // quads, and the slices left (a list of one side as the same stack in the
+        // other drivers).  One set of quads, and one set of single
         // slices per distinct schedule, in the order of each schedule's
         // largest side.
         struct Item {
             int at, n, quad;                   // first place in `order`, slices, held as one quad
         };
         std::vector<Item> items;
+        const bool alike = slices[order[0]].n == slices[order[count - 1]].n;
         long long qblocks = 0, qbp = 0, left = 0;
         for (int pass = 0; pass < 2; ++pass) {
-            const bool use = pass == 1 && qbp >= QUAD_MIN_BP_BLOCKS &&
-                             quads_fill(qblocks, left > 0 ? QUAD_MIN_BLOCKS_BESIDE_SINGLES : QUAD_MIN_BLOCKS);
+            const bool use = pass == 1 && (alike || (qbp >= QUAD_MIN_BP_BLOCKS &&
+                             quads_fill(qblocks, left > 0 ? QUAD_MIN_BLOCKS_BESIDE_SINGLES : QUAD_MIN_BLOCKS)));
             items.clear();
             for (int r = 0; r < count;) {
                 const int n = slices[order[r]].n;
                 int e = r;
                 while (e < count && slices[order[e]].n == n) ++e;
-                const int nq = quads_allowed(c, n) && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS ? quad_part(e - r) : 0;
+                int nq = 0;
+                if (quads_allowed(c, n) && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS)
+                    nq = alike ? quads_of(count, n, fp_quad_blocks(n, na), bp_blocks(n, n, QBP_ROWS)) : quad_part(e - r);
                 if (pass == 0) {
                     left += e - r - nq;
                     qblocks += (long long)nq * fp_quad_blocks(n, na);
@@ -2357,10 +2406,9 @@ ctr_status align_forward(ctr_ctx *c, const float *img, const float *shifts, floa
     StackBind b;
     b.src = img;
     std::vector<SliceSet *> sets;
-    const int D = std::max(g.nx, g.ny), part = quad_part(dN);
-    const bool quads = D <= LDS_FP_MAX_SIDE && quads_fill((long long)part * fp_quad_blocks(g.px, g.pa), ALIGN_QUAD_MIN_BLOCKS) &&
-                       rim_texels(c, D, 1) <= QUAD_MAX_RIM_TEXELS;
-    const int nq = quads ? part : 0;
+    const int D = std::max(g.nx, g.ny);
+    int nq = D <= LDS_FP_MAX_SIDE ? align_quads_of(dN, D, fp_quad_blocks(g.px, g.pa)) : 0;
+    if (nq > 0 && !(rim_texels(c, D, 1) <= QUAD_MAX_RIM_TEXELS)) nq = 0;
     TRY(split_stack(c, dN, nq, false, b, sets));
     for (SliceSet *S : sets) {
         TRY(run_kind(c, *S, G_PAD));
