@@ -814,27 +814,54 @@ double rim_texels(const ctr_ctx *c, int D, int stride)
 // Whether one slice left over of side D joins as a quad (of per_quad projection blocks).
 bool one_joins(int D, int per_quad) { return D <= QUAD_ONE_OVER_SIDE && (long long)per_quad * D <= QUAD_ONE_OVER_WORK; }
 
-// How many of n equal slices of side D run as quads where they are all there is.
-// per_quad, bp_per_quad: a quad's projection and backprojection blocks.
-int quads_of(int n, int D, int per_quad, int bp_per_quad)
+// The part of a slice's projection blocks that have work.  Rays beyond the image have
+// none, and across a long and narrow image few of them have much: those blocks count
+// in a launch of single slices, which has eight times as many, but not here.  Quads
+// against single slices, us per subset of a call of four: 8 x 284^2 with 1136 bins, 60
+// angles, 1.30 times their time, 4 x 364^2 with 2184, 60, 1.41, 8 x 424^2 with 1060, 60,
+// 1.14, 16 x 241^2 with 964, 60, 1.00, 24 x 281^2 with 1124, 40, 0.82; 12 x 1253 x 98 with
+// 1253, 40, 1.27, 8 x 2048 x 64 with 2048, 60, 1.85, 4 x 120 x 1296 with 1296, 130, 1.02,
+// 32 x 817 x 145 with 817, 40, 0.73.  wide: the power of the image's share of the
+// detector; the alignment forward (1) loses more: 4 x 533^2 with 2132, 120 angles 1.56,
+// 8 x 416^2 with 1664, 120, 1.14.
+double live_share(int nx, int ny, int px, double wide)
 {
-    if (n < QZ - 1) return 0;
+    const double D = std::max(nx, ny), d = std::min(nx, ny);
+    return std::pow(std::min(1.0, D / px), wide) * std::min(1.0, 3.0 * d / D);
+}
+constexpr double STACK_WIDE = 0.7, ALIGN_WIDE = 1.0;
+
+}  // namespace
+
+int ctr::stack_quads_of(int n, int nx, int ny, int px, int na)
+{
+    const int D = std::max(nx, ny), per_quad = fp_quad_blocks(px, na);
+    if (n < QZ - 1 || D > LDS_FP_MAX_SIDE) return 0;
     const bool one = n % QZ == 1;
     const int nq = one && !one_joins(D, per_quad) ? n - 1 : n;
     const long long least = !one ? QUAD_MIN_BLOCKS : (D <= QUAD_ONE_OVER_SIDE ? QUAD_MIN_BLOCKS_ONE_SMALL : QUAD_MIN_BLOCKS_ONE_LARGE);
-    return quads_fill((long long)nq * per_quad, least) && (long long)((nq + QZ - 1) / QZ) * bp_per_quad >= QUAD_MIN_BP_BLOCKS
+    return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, STACK_WIDE)), least) &&
+                   (long long)((nq + QZ - 1) / QZ) * bp_blocks(nx, ny, QBP_ROWS) >= QUAD_MIN_BP_BLOCKS
                ? nq : 0;
 }
 
-// The same for the layers of an alignment forward.
-int align_quads_of(int n, int D, int per_quad)
+int ctr::align_quads_of(int n, int nx, int ny, int px, int pa)
 {
-    if (n < QZ - 1) return 0;
+    const int D = std::max(nx, ny), per_quad = fp_quad_blocks(px, pa);
+    if (n < QZ - 1 || D > LDS_FP_MAX_SIDE) return 0;
     const bool one = n % QZ == 1, in = one && n > 2 * QZ && one_joins(D, per_quad);
     const int nq = one && !in ? n - 1 : n;
     const long long least = in ? ALIGN_QUAD_MIN_BLOCKS_ONE_IN : (one ? ALIGN_QUAD_MIN_BLOCKS_ONE_BESIDE : ALIGN_QUAD_MIN_BLOCKS);
-    return quads_fill((long long)nq * per_quad, least) ? nq : 0;
+    return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, ALIGN_WIDE)), least) ? nq : 0;
 }
+
+int ctr::fbp_quads_of(int n, int nx, int ny, int zp)
+{
+    const int nq = quad_part(n);
+    return (long long)((nq + QZ - 1) / QZ) * fbp_quad_blocks(nx, ny) >= FBP_QUAD_MIN_BLOCKS && zp <= FBP_QUAD_MAX_ZP ? nq : 0;
+}
+
+namespace {
 
 // Layers of a uniform stack of nz that the subset drivers run as quads.
 int stack_quads(ctr_ctx *c, int nz)
@@ -842,7 +869,7 @@ int stack_quads(ctr_ctx *c, int nz)
     const ctr_geometry &g = c->g;
     const int D = std::max(g.nx, g.ny);
     if (!quads_allowed(c, D)) return 0;
-    const int nq = quads_of(nz, D, fp_quad_blocks(g.px, g.pa / g.ss), bp_blocks(g.nx, g.ny, QBP_ROWS));
+    const int nq = stack_quads_of(nz, g.nx, g.ny, g.px, g.pa / g.ss);
     return nq > 0 && rim_texels(c, D, g.ss) <= QUAD_MAX_RIM_TEXELS ? nq : 0;
 }
 
@@ -1423,8 +1450,7 @@ extern "C" ctr_status ctr_fbp_execution(ctr_ctx *c, float *img, float *prj, int 
     const Layout l = make_layout(g.nx, g.ny, g.px);
     // whole quads of layers (and two or three left over) filter and
     // backproject interleaved, the others singly
-    int nq = quad_part(dN);
-    if ((long long)((nq + QZ - 1) / QZ) * fbp_quad_blocks(g.nx, g.ny) < FBP_QUAD_MIN_BLOCKS || g.zp > FBP_QUAD_MAX_ZP) nq = 0;
+    const int nq = fbp_quads_of(dN, g.nx, g.ny, g.zp);
     const size_t qrows = (size_t)((nq + QZ - 1) / QZ) * QZ, row = (size_t)g.pa * l.rpitch;
     HIPTRY(c, c->w_rows.ensure(sizeof(float) * (qrows + (size_t)(dN - nq)) * row));
     if (prj_correction && g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
@@ -2056,7 +2082,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
                 while (e < count && slices[order[e]].n == n) ++e;
                 int nq = 0;
                 if (quads_allowed(c, n) && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS)
-                    nq = alike ? quads_of(count, n, fp_quad_blocks(n, na), bp_blocks(n, n, QBP_ROWS)) : quad_part(e - r);
+                    nq = alike ? stack_quads_of(count, n, n, n, na) : quad_part(e - r);
                 if (pass == 0) {
                     left += e - r - nq;
                     qblocks += (long long)nq * fp_quad_blocks(n, na);
@@ -2407,7 +2433,7 @@ ctr_status align_forward(ctr_ctx *c, const float *img, const float *shifts, floa
     b.src = img;
     std::vector<SliceSet *> sets;
     const int D = std::max(g.nx, g.ny);
-    int nq = D <= LDS_FP_MAX_SIDE ? align_quads_of(dN, D, fp_quad_blocks(g.px, g.pa)) : 0;
+    int nq = align_quads_of(dN, g.nx, g.ny, g.px, g.pa);
     if (nq > 0 && !(rim_texels(c, D, 1) <= QUAD_MAX_RIM_TEXELS)) nq = 0;
     TRY(split_stack(c, dN, nq, false, b, sets));
     for (SliceSet *S : sets) {

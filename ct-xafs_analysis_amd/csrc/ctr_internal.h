@@ -149,6 +149,10 @@ void launch_fbp_filter(const float *prj, float *frows, int nz, int pa, int px, i
 constexpr long long FBP_QUAD_MIN_BLOCKS = 512;
 // A quad's filter block holds two transforms (16 ZP bytes of LDS).
 constexpr int FBP_QUAD_MAX_ZP = 4096;
+// The backprojection kernel of a call over `units` slices or quads: slices side by
+// side, rows, angle shares.
+enum FbpKernel { FBP_1_4_8 = 148, FBP_1_8_4 = 184, FBP_1_4_0 = 140, FBP_4_4_4 = 444, FBP_4_4_0 = 440 };
+int fbp_kernel(int nx, int ny, int units, int quads);
 void launch_fbp_bp(const float *frows, float *img, const float2 *cs, int nz, int nx, int ny, int pa,
                    int px, int rpitch, int roff, int quads, hipStream_t stream);
 void launch_rows_to_full(const float *rows, float *full, int nz, int na, int rpitch, int roff, int pa, int px,
@@ -175,6 +179,12 @@ void launch_align_adjoint(const float *prj, float *gpad, const float2 *cs, const
 void launch_align_grad(const float *pimg, const float *pimgT, int ipitch, int tpitch, const float2 *cs,
                        const float *gprj, const float *shifts, float center, float *partial, float *gshift,
                        int nz, int nx, int ny, int pa, int px, hipStream_t stream);
+
+// How many of n equal slices run as quads where they are all there is: layers of an
+// OS-EM, TV OS-EM or AART stack (na angles a subset), of an alignment forward, of FBP.
+int stack_quads_of(int n, int nx, int ny, int px, int na);
+int align_quads_of(int n, int nx, int ny, int px, int pa);
+int fbp_quads_of(int n, int nx, int ny, int zp);
 
 // blocks per slice for each grid kind
 int fp_blocks(int px, int na, int wpb, int rays);
