@@ -788,6 +788,13 @@ constexpr long long ALIGN_QUAD_MIN_BLOCKS_ONE_IN = 1200, ALIGN_QUAD_MIN_BLOCKS_O
 // images with many angles need this many of them: 32 x 128^2, 90 angles (128) 55
 // us a subset and 58 as single slices; 8 x 131^2, 261 angles (54) 100 and 76.
 constexpr long long QUAD_MIN_BP_BLOCKS = 112;
+// AART begins with a backprojection of the sinograms themselves, whose gathers quads
+// with few blocks hide worse: in calls of few subsets in all they need more.  One
+// iteration of two subsets, us per subset: 16 x 147^2, 180 angles (120 blocks) 200 /
+// 144; 16 x 204^2, 700 (208) 1.08 times the single slices' time; 24 x 194^2, 90 (312)
+// 1.05; 16 x 273^2, 180 (360) 261 / 289.
+constexpr int QUAD_INIT_PASSES = 16;
+constexpr long long QUAD_MIN_BP_BLOCKS_INIT = 320;
 // The two angles of a quad's projection block share a window while the rims of
 // their strips lie close: 21 x 1221^2, 23 angles (83 texels) take 1.25 times the
 // single slices' time, 4 x 2048^2, 40 angles (80) 0.96, 4 x 1536^2, 60 angles (40)
@@ -821,27 +828,28 @@ bool one_joins(int D, int per_quad) { return D <= QUAD_ONE_OVER_SIDE && (long lo
 // angles, 1.30 times their time, 4 x 364^2 with 2184, 60, 1.41, 8 x 424^2 with 1060, 60,
 // 1.14, 16 x 241^2 with 964, 60, 1.00, 24 x 281^2 with 1124, 40, 0.82; 12 x 1253 x 98 with
 // 1253, 40, 1.27, 8 x 2048 x 64 with 2048, 60, 1.85, 4 x 120 x 1296 with 1296, 130, 1.02,
-// 32 x 817 x 145 with 817, 40, 0.73.  wide: the power of the image's share of the
-// detector; the alignment forward (1) loses more: 4 x 533^2 with 2132, 120 angles 1.56,
-// 8 x 416^2 with 1664, 120, 1.14.
-double live_share(int nx, int ny, int px, double wide)
+// 32 x 817 x 145 with 817, 40, 0.73; 8 x 752^2 with 3008, 24, 1.64, 16 x 778^2 with 4668,
+// 24, 0.89.  wide: the power of the image's share of the detector, slim: how much
+// longer than wide an image may be before it counts.
+double live_share(int nx, int ny, int px, double wide, double slim)
 {
     const double D = std::max(nx, ny), d = std::min(nx, ny);
-    return std::pow(std::min(1.0, D / px), wide) * std::min(1.0, 3.0 * d / D);
+    return std::pow(std::min(1.0, D / px), wide) * std::min(1.0, slim * d / std::min(D, (double)px));
 }
-constexpr double STACK_WIDE = 0.7, ALIGN_WIDE = 1.0;
 
 }  // namespace
 
-int ctr::stack_quads_of(int n, int nx, int ny, int px, int na)
+int ctr::stack_quads_of(int n, int nx, int ny, int px, int na, int passes)
 {
     const int D = std::max(nx, ny), per_quad = fp_quad_blocks(px, na);
     if (n < QZ - 1 || D > LDS_FP_MAX_SIDE) return 0;
     const bool one = n % QZ == 1;
     const int nq = one && !one_joins(D, per_quad) ? n - 1 : n;
     const long long least = !one ? QUAD_MIN_BLOCKS : (D <= QUAD_ONE_OVER_SIDE ? QUAD_MIN_BLOCKS_ONE_SMALL : QUAD_MIN_BLOCKS_ONE_LARGE);
-    return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, STACK_WIDE)), least) &&
-                   (long long)((nq + QZ - 1) / QZ) * bp_blocks(nx, ny, QBP_ROWS) >= QUAD_MIN_BP_BLOCKS
+    const double share = live_share(nx, ny, px, D <= QUAD_ONE_OVER_SIDE ? 0.7 : 1.0, 3.0);
+    const long long bp = passes < QUAD_INIT_PASSES ? QUAD_MIN_BP_BLOCKS_INIT : QUAD_MIN_BP_BLOCKS;
+    return quads_fill((long long)((double)nq * per_quad * share), least) &&
+                   (long long)((nq + QZ - 1) / QZ) * bp_blocks(nx, ny, QBP_ROWS) >= bp
                ? nq : 0;
 }
 
@@ -850,9 +858,16 @@ int ctr::align_quads_of(int n, int nx, int ny, int px, int pa)
     const int D = std::max(nx, ny), per_quad = fp_quad_blocks(px, pa);
     if (n < QZ - 1 || D > LDS_FP_MAX_SIDE) return 0;
     const bool one = n % QZ == 1, in = one && n > 2 * QZ && one_joins(D, per_quad);
+    // on a detector this wide quads gain nothing that could pay for one layer more: 8 and
+    // 9 of 284^2 with 738 bins, 1123 angles 714 / 676 and 893 / 772; with 430 438 / 566
+    // and 552 / 650
+    if (one && px > 2 * D) return 0;
     const int nq = one && !in ? n - 1 : n;
     const long long least = in ? ALIGN_QUAD_MIN_BLOCKS_ONE_IN : (one ? ALIGN_QUAD_MIN_BLOCKS_ONE_BESIDE : ALIGN_QUAD_MIN_BLOCKS);
-    return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, ALIGN_WIDE)), least) ? nq : 0;
+    // 12 x 198^2 with 792 bins, 60 angles (1170 blocks) 94 / 87; 16 x 274^2 with 465, 60
+    // (960) 134 / 112; 12 x 861 x 80 with 861, 60 (1260) 151 / 131; 6 x 113^2 with 282, 900
+    // (3375) 160 / 172; 8 x 241 x 34 with 111, 812 (1624) 82 / 119.
+    return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, 0.3, 5.0)), least) ? nq : 0;
 }
 
 int ctr::fbp_quads_of(int n, int nx, int ny, int zp)
@@ -863,13 +878,14 @@ int ctr::fbp_quads_of(int n, int nx, int ny, int zp)
 
 namespace {
 
-// Layers of a uniform stack of nz that the subset drivers run as quads.
-int stack_quads(ctr_ctx *c, int nz)
+// Layers of a uniform stack of nz that the subset drivers run as quads.  passes:
+// subsets of the call, for drivers that begin with a backprojection of their own.
+int stack_quads(ctr_ctx *c, int nz, int passes = INT_MAX)
 {
     const ctr_geometry &g = c->g;
     const int D = std::max(g.nx, g.ny);
     if (!quads_allowed(c, D)) return 0;
-    const int nq = stack_quads_of(nz, g.nx, g.ny, g.px, g.pa / g.ss);
+    const int nq = stack_quads_of(nz, g.nx, g.ny, g.px, g.pa / g.ss, passes);
     return nq > 0 && rim_texels(c, D, g.ss) <= QUAD_MAX_RIM_TEXELS ? nq : 0;
 }
 
@@ -1417,7 +1433,8 @@ extern "C" ctr_status ctr_aart_execution(ctr_ctx *c, float *img, float *prj, int
     StackBind b;
     b.prj = prj; b.src = img; b.dst = img;
     std::vector<SliceSet *> sets;
-    TRY(split_stack(c, dN, stack_quads(c, dN), true, b, sets));
+    const int passes = (int)std::min((long long)INT_MAX, (long long)g.ss * std::max(it, 0));
+    TRY(split_stack(c, dN, stack_quads(c, dN, passes), true, b, sets));
     if (g.correction_mode > 0) TRY(correct_in_place(c, prj, dN));
     for (SliceSet *S : sets) {
         // zero borders of both copies (the interior is overwritten next)
@@ -2082,7 +2099,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
                 while (e < count && slices[order[e]].n == n) ++e;
                 int nq = 0;
                 if (quads_allowed(c, n) && rim_texels(c, n, c->g.ss) <= QUAD_MAX_RIM_TEXELS)
-                    nq = alike ? stack_quads_of(count, n, n, n, na) : quad_part(e - r);
+                    nq = alike ? stack_quads_of(count, n, n, n, na, INT_MAX) : quad_part(e - r);
                 if (pass == 0) {
                     left += e - r - nq;
                     qblocks += (long long)nq * fp_quad_blocks(n, na);

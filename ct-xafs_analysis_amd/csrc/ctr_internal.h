@@ -181,8 +181,9 @@ void launch_align_grad(const float *pimg, const float *pimgT, int ipitch, int tp
                        int nz, int nx, int ny, int pa, int px, hipStream_t stream);
 
 // How many of n equal slices run as quads where they are all there is: layers of an
-// OS-EM, TV OS-EM or AART stack (na angles a subset), of an alignment forward, of FBP.
-int stack_quads_of(int n, int nx, int ny, int px, int na);
+// OS-EM, TV OS-EM or AART stack (na angles a subset; passes: subsets in all for AART,
+// else INT_MAX), of an alignment forward, of FBP.
+int stack_quads_of(int n, int nx, int ny, int px, int na, int passes);
 int align_quads_of(int n, int nx, int ny, int px, int pa);
 int fbp_quads_of(int n, int nx, int ny, int zp);
 

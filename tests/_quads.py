@@ -15,9 +15,10 @@ def rim_texels(ang, D, stride):
     return float(step.mean() * np.pi / 180.0 * 0.5 * D) if len(a) > 1 else 0.0
 
 
-def stack_quads(nx, ny, px, pa, ss, dn, ang):
-    """Layers of an OS-EM, TV OS-EM or AART stack that run as quads."""
-    nq = _LIB._ZN3ctr14stack_quads_ofEiiiii(dn, nx, ny, px, pa // ss)
+def stack_quads(nx, ny, px, pa, ss, dn, ang, passes=2 ** 31 - 1):
+    """Layers of an OS-EM, TV OS-EM or AART (passes: its subsets in all) stack that run
+    as quads."""
+    nq = _LIB._ZN3ctr14stack_quads_ofEiiiiii(dn, nx, ny, px, pa // ss, passes)
     return nq if nq and rim_texels(ang, max(nx, ny), ss) <= MAX_RIM_TEXELS else 0
 
 

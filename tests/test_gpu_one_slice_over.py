@@ -57,8 +57,15 @@ def test_one_slice_over(ctx, n, px, na, dn, nq):
         one = dev(x0[z:z + 1])
         ctx.osem_execution(one, y[z:z + 1].contiguous(), 1)
         assert np.array_equal(host(one)[0], got[z]), z
-    xa = dev(x0)
-    assert _launches(ctx, lambda: ctx.aart_execution(xa, y.clone(), 1)) == parts
+    for it in (1, 16):                           # AART of few subsets needs more blocks
+        nqa = _quads.stack_quads(n, n, px, na, 1, dn, ang, passes=it)
+        xa = dev(x0)
+        assert _launches(ctx, lambda: ctx.aart_execution(xa, y.clone(), it)) == it * ((nqa > 0) + (nqa < dn))
+        for z in (0, dn - 1):
+            one = dev(x0[z:z + 1])
+            ctx.aart_execution(one, y[z:z + 1].clone(), it)
+            assert np.array_equal(host(one)[0], host(xa)[z]), (it, z)
+    assert nqa == nq
     if px == n:                                  # a batch's detector is its side
         imgs = [dev(v) for v in x0]
         assert _launches(ctx, lambda: ctx.osem_batched(imgs, [y[z] for z in range(dn)], 1, use_graph=False)) == parts
@@ -67,7 +74,7 @@ def test_one_slice_over(ctx, n, px, na, dn, nq):
 
 @pytest.mark.parametrize("n,px,pa,dn,nq", [
     (128, 128, 900, 5, 0), (130, 65, 903, 9, 9), (520, 512, 400, 5, 4), (256, 256, 340, 9, 9), (256, 256, 200, 9, 0),
-    (256, 256, 700, 9, 8)])
+    (256, 256, 700, 9, 8), (33, 400, 900, 4, 4)])
 @pytest.mark.parametrize("deriv", [False, True])
 def test_one_layer_over_in_the_alignment_forward(ctx, n, px, pa, dn, nq, deriv):
     """Equal to one layer at a time, with offsets, and NaN for an angle whose offset is
