@@ -781,7 +781,10 @@ constexpr long long QUAD_MIN_BLOCKS_BESIDE_SINGLES = 1800;
 // without it) 196 / 189 / 182; 5 x 512^2, 300 (1200) - / 261 / 259, without the
 // derivative - / 230 / 237; 5 x 512^2, 400 (1600) 340 / 297 / 325; 5 x 742^2, 200 (1200)
 // 367 / 352 / 341.
-constexpr long long ALIGN_QUAD_MIN_BLOCKS = 800;
+// With two over, in a quad with two empty places: 6 x 398^2, 243 angles (1281 blocks of
+// 1708) 203 / 189; 6 x 716^2, 120 (1080) 274 / 267; 6 x 608^2 with 425 bins, 250 (1312) 271
+// / 278.
+constexpr long long ALIGN_QUAD_MIN_BLOCKS = 800, ALIGN_QUAD_MIN_BLOCKS_TWO_OVER = 1300;
 constexpr long long ALIGN_QUAD_MIN_BLOCKS_ONE_IN = 1200, ALIGN_QUAD_MIN_BLOCKS_ONE_BESIDE = 1200;
 
 // A quad's backprojection sums all angles of 64 x 16 pixels in one block, so small
@@ -792,8 +795,9 @@ constexpr long long QUAD_MIN_BP_BLOCKS = 112;
 // with few blocks hide worse: in calls of few subsets in all they need more.  One
 // iteration of two subsets, us per subset: 16 x 147^2, 180 angles (120 blocks) 200 /
 // 144; 16 x 204^2, 700 (208) 1.08 times the single slices' time; 24 x 194^2, 90 (312)
-// 1.05; 16 x 273^2, 180 (360) 261 / 289.
-constexpr int QUAD_INIT_PASSES = 16;
+// 1.05; 16 x 273^2, 180 (360) 261 / 289.  Ten subsets, 32 x 128^2 with 1024 bins, 60 (128)
+// 78 / 90.
+constexpr int QUAD_INIT_PASSES = 8;
 constexpr long long QUAD_MIN_BP_BLOCKS_INIT = 320;
 // The two angles of a quad's projection block share a window while the rims of
 // their strips lie close: 21 x 1221^2, 23 angles (83 texels) take 1.25 times the
@@ -863,11 +867,12 @@ int ctr::align_quads_of(int n, int nx, int ny, int px, int pa)
     // and 552 / 650
     if (one && px > 2 * D) return 0;
     const int nq = one && !in ? n - 1 : n;
-    const long long least = in ? ALIGN_QUAD_MIN_BLOCKS_ONE_IN : (one ? ALIGN_QUAD_MIN_BLOCKS_ONE_BESIDE : ALIGN_QUAD_MIN_BLOCKS);
+    const long long least = in ? ALIGN_QUAD_MIN_BLOCKS_ONE_IN : (one ? ALIGN_QUAD_MIN_BLOCKS_ONE_BESIDE : (n % QZ == 2 ? ALIGN_QUAD_MIN_BLOCKS_TWO_OVER : ALIGN_QUAD_MIN_BLOCKS));
     // 12 x 198^2 with 792 bins, 60 angles (1170 blocks) 94 / 87; 16 x 274^2 with 465, 60
     // (960) 134 / 112; 12 x 861 x 80 with 861, 60 (1260) 151 / 131; 6 x 113^2 with 282, 900
-    // (3375) 160 / 172; 8 x 241 x 34 with 111, 812 (1624) 82 / 119.
-    return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, 0.3, 5.0)), least) ? nq : 0;
+    // (3375) 160 / 172; 4 x 256^2 with 2048, 100 (1600) 114 / 81; 8 x 241 x 34 with 111, 812
+    // (1624) 82 / 119.
+    return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, 0.5, 5.0)), least) ? nq : 0;
 }
 
 int ctr::fbp_quads_of(int n, int nx, int ny, int zp)

@@ -13,13 +13,13 @@ def _angles(pa):
     return (np.arange(pa) * (180.0 / pa)).astype(np.float32)
 
 
-QUADS = [c + (8,) for c in CASES[:3]] + [(193, 130, 180, 108, 3, 46, 1)]       # the last by its blocks
+QUADS = [c + (4,) for c in CASES[:3]] + [(193, 130, 180, 108, 3, 46, 1)]       # the last by its blocks
 
 
 def test_they_run_as_quads():
     for nx, ny, px, pa, ss, dn, it in QUADS:
         assert _quads.stack_quads(nx, ny, px, pa, ss, dn, _angles(pa), passes=ss * it) >= dn - 1
-        assert ss * it >= 16 or (nx, ny) == (193, 130)
+        assert ss * it >= 8 or (nx, ny) == (193, 130)
     nx, ny, px, pa, ss, dn = CASES[0]
     assert _quads.stack_quads(nx, ny, px, pa, ss, dn, _angles(pa), passes=ss * 2) == 0
 

@@ -57,7 +57,7 @@ def test_one_slice_over(ctx, n, px, na, dn, nq):
         one = dev(x0[z:z + 1])
         ctx.osem_execution(one, y[z:z + 1].contiguous(), 1)
         assert np.array_equal(host(one)[0], got[z]), z
-    for it in (1, 16):                           # AART of few subsets needs more blocks
+    for it in (1, 8):                           # AART of few subsets needs more blocks
         nqa = _quads.stack_quads(n, n, px, na, 1, dn, ang, passes=it)
         xa = dev(x0)
         assert _launches(ctx, lambda: ctx.aart_execution(xa, y.clone(), it)) == it * ((nqa > 0) + (nqa < dn))

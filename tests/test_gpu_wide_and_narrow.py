@@ -48,6 +48,9 @@ def test_alignment_forward_counts_the_same():
     assert _quads.align_quads(198, 198, 792, 60, 12, ang[::2]) == 0
     assert _quads.align_quads(1197, 116, 1197, 120, 4, ang) == 0
     assert _quads.align_quads(241, 34, 111, 812, 8, _angles(812)) == 8
+    assert _quads.align_quads(398, 398, 398, 243, 6, _angles(243)) == 0
+    assert _quads.align_quads(398, 398, 398, 243, 8, _angles(243)) == 8
+    assert _quads.align_quads(256, 256, 2048, 100, 4, _angles(100)) == 0
     assert _quads.align_quads(284, 284, 738, 1123, 9, _angles(1123)) == 0
     assert _quads.align_quads(284, 284, 430, 1123, 9, _angles(1123)) == 8
     assert _quads.align_quads(533, 533, 533, 240, 4, ang) == 4
