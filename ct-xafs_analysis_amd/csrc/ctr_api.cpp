@@ -765,11 +765,15 @@ constexpr long long QUAD_MIN_BLOCKS = 560;
 constexpr int QUAD_ONE_OVER_SIDE = 512;
 constexpr long long QUAD_ONE_OVER_WORK = 350000;
 constexpr long long QUAD_MIN_BLOCKS_ONE_SMALL = 900, QUAD_MIN_BLOCKS_ONE_LARGE = 640;
-// The same for batches of several sides that also leave single slices, whose launches
-// come on top: 41 slices of 189^2 to 511^2, 42 angles (929 blocks) 1.21 ms a call with
-// quads and 1.02 all single; 30 of 185^2 to 1109^2, 62 angles (1270) 24.0 and 21.8;
-// 59 of 255^2 to 1024^2, 120 angles (over 5000) 11.9, and 20.1 with the single
-// slices' kernels of before.
+// The same for batches of several sides, whose blocks differ in length.  Single slices
+// against quads, both of 2 to 9 sides, the ratio of their times: 10 x 140^2, 8 x 588^2 and 3
+// x 837^2, 30 angles (570 blocks) 0.89; 6 x 135^2, 4 x 137^2, 3 x 1003^2, 62 (604) 0.86;
+// 11 x 140^2, 8 x 212^2, 90 (731) 0.94; 8 x 445^2, 12 x 524^2, 4 x 713^2, 30 (795) 1.07; 7 x
+// 150^2, 10 x 154^2, 12 x 548^2, 42 (834) 1.06; 12 x 248^2, 7 x 374^2, 90 (1012) 1.09.  Lists
+// that also leave single slices, whose launches come on top, 70 at random: 31 below
+// 1000 blocks at 0.71 to 1.11, 31 from there to 1800 at 0.91 to 1.19 (six below 1), 8
+// beyond at 1.04 to 1.31.
+constexpr long long QUAD_MIN_BLOCKS_UNEVEN = 780;
 constexpr long long QUAD_MIN_BLOCKS_BESIDE_SINGLES = 1800;
 // The same for the alignment forward with its derivative, whose quads take longer:
 // 4 x 128^2, 900 angles (900) 81 / 96; 4 x 512^2, 225 (904) 163 / 184; 4 x 1024^2,
@@ -873,6 +877,11 @@ int ctr::align_quads_of(int n, int nx, int ny, int px, int pa)
     // (3375) 160 / 172; 4 x 256^2 with 2048, 100 (1600) 114 / 81; 8 x 241 x 34 with 111, 812
     // (1624) 82 / 119.
     return quads_fill((long long)((double)nq * per_quad * live_share(nx, ny, px, 0.5, 5.0)), least) ? nq : 0;
+}
+
+bool ctr::batch_takes_quads(long long blocks, long long bp, long long left)
+{
+    return bp >= QUAD_MIN_BP_BLOCKS && quads_fill(blocks, left > 0 ? QUAD_MIN_BLOCKS_BESIDE_SINGLES : QUAD_MIN_BLOCKS_UNEVEN);
 }
 
 int ctr::fbp_quads_of(int n, int nx, int ny, int zp)
@@ -2095,8 +2104,7 @@ extern "C" ctr_status ctr_osem_batched(ctr_ctx *c, const ctr_slice *slices, int 
         const bool alike = slices[order[0]].n == slices[order[count - 1]].n;
         long long qblocks = 0, qbp = 0, left = 0;
         for (int pass = 0; pass < 2; ++pass) {
-            const bool use = pass == 1 && (alike || (qbp >= QUAD_MIN_BP_BLOCKS &&
-                             quads_fill(qblocks, left > 0 ? QUAD_MIN_BLOCKS_BESIDE_SINGLES : QUAD_MIN_BLOCKS)));
+            const bool use = pass == 1 && (alike || batch_takes_quads(qblocks, qbp, left));
             items.clear();
             for (int r = 0; r < count;) {
                 const int n = slices[order[r]].n;

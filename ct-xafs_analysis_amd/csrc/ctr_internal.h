@@ -186,6 +186,10 @@ void launch_align_grad(const float *pimg, const float *pimgT, int ipitch, int tp
 int stack_quads_of(int n, int nx, int ny, int px, int na, int passes);
 int align_quads_of(int n, int nx, int ny, int px, int pa);
 int fbp_quads_of(int n, int nx, int ny, int zp);
+// Whether the equal slices of a batch of several sides run as quads: blocks, the
+// projection blocks of all quads, each times the slices it holds; bp, their
+// backprojection blocks; left, the slices that would stay single.
+bool batch_takes_quads(long long blocks, long long bp, long long left);
 
 // blocks per slice for each grid kind
 int fp_blocks(int px, int na, int wpb, int rays);

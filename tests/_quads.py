@@ -1,5 +1,7 @@
 """The library's choice between quads (four slices side by side) and single slices:
 its own functions, called on the host, and the distance of the angles restated."""
+import ctypes
+
 import numpy as np
 import torch  # noqa: F401  (its HIP runtime is the one to load first)
 from ctrecon import load
@@ -34,3 +36,18 @@ def fbp_kernels(nx, ny, zp, dn):
     nq = _LIB._ZN3ctr12fbp_quads_ofEiiii(dn, nx, ny, zp)
     parts = [((nq + 3) // 4, 1)] * (nq > 0) + [(dn - nq, 0)] * (nq < dn)
     return nq, {_LIB._ZN3ctr10fbp_kernelEiiii(nx, ny, units, quads) for units, quads in parts}
+
+
+def batch_quads(sides, na):
+    """Slices of a batch that run as quads (angles close enough to share windows)."""
+    runs = {n: sides.count(n) for n in set(sides)}
+    if len(runs) == 1:
+        n = sides[0]
+        return _LIB._ZN3ctr14stack_quads_ofEiiiiii(len(sides), n, n, n, na, 2 ** 31 - 1)
+    part = {n: k if k >= 3 and k % 4 >= 2 else k // 4 * 4 for n, k in runs.items()}
+    blocks = sum(q * ((n + 63) // 64) * ((na + 1) // 2) for n, q in part.items())
+    bp = sum((q + 3) // 4 * ((n + 63) // 64) * ((n + 15) // 16) for n, q in part.items())
+    nq = sum(part.values())
+    take = _LIB._ZN3ctr17batch_takes_quadsExxx
+    take.argtypes, take.restype = [ctypes.c_longlong] * 3, ctypes.c_bool
+    return nq if take(blocks, bp, len(sides) - nq) else 0
