@@ -967,6 +967,8 @@ void time_end(ctr_ctx *c, int which)
 ctr_status run_fp(ctr_ctx *c, SliceSet &S, int var, int sub, int sub_from_layer, int geo_power)
 {
     FpParams p{sub, c->g.ss, c->g.pa / c->g.ss, sub_from_layer, geo_power, 0};
+    if (S.quad && (sub_from_layer || geo_power || var == FP_RAW))
+        return fail(c, CTR_NOT_SUPPORTED, "quads project the subset drivers' subsets only");
     time_begin(c, 0);
     if (S.quad) launch_fp_quad(var, launch_of(c, S, G_FP), p, c->stream);
     else launch_fp(var, S.fp_wpb, S.fp_rays, S.fp_tile, launch_of(c, S, G_FP), p, c->stream);
@@ -979,6 +981,8 @@ ctr_status run_bp(ctr_ctx *c, SliceSet &S, int var, int sub, int sub_from_layer,
                   int to_aux, int write_t = 0)
 {
     BpParams p{sub, c->g.ss, c->g.pa / c->g.ss, c->g.pa, sub_from_layer, alpha, L, to_aux, 0, write_t};
+    if (S.quad && (sub_from_layer || (var != BP_OSEM2 && var != BP_AART2 && var != BP_INIT)))
+        return fail(c, CTR_NOT_SUPPORTED, "quads backproject the subset drivers' subsets only");
     time_begin(c, 1);
     if (S.quad) launch_bp_quad(var, launch_of(c, S, G_BP), p, c->stream);
     else launch_bp(var, S.bp_rows, launch_of(c, S, G_BP), p, c->stream);

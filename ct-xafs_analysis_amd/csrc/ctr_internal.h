@@ -85,7 +85,8 @@ struct BpParams {
 // ---- launchers (ctr_kernels.hip) ----
 void launch_fp(int var, int wpb, int rays, int tile, const Launch &L, const FpParams &p, hipStream_t stream);
 void launch_bp(int var, int rows, const Launch &L, const BpParams &p, hipStream_t stream);
-// The same over quads (a set of quads only; LDS-tiled projector).
+// The same over quads (a set of quads only; LDS-tiled projector): FP_RATIO and
+// FP_RESID; BP_OSEM2, BP_AART2 and BP_INIT, of one subset for all slices.
 void launch_fp_quad(int var, const Launch &L, const FpParams &p, hipStream_t stream);
 void launch_bp_quad(int var, const Launch &L, const BpParams &p, hipStream_t stream);
 void launch_pad_quad(const Launch &L, hipStream_t stream);     // src planes -> both padded copies

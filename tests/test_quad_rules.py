@@ -1,11 +1,9 @@
 """The choice between quads and single slices, from the library's own functions on the
-host: stacks that the GPU tests mean to run as quads do so, the FBP tests between
-them reach every backprojection kernel, and batches of several sides stay single
-where quads would lose."""
+host: stacks that the GPU tests mean to run as quads do so, and batches of several
+sides stay single where quads would lose."""
 import numpy as np
 
 import _quads
-import test_gpu_align_quads
 import test_gpu_coupled_stacks
 import test_gpu_quads
 from test_gpu_quads import _angles
