@@ -575,9 +575,9 @@ def main():
     tune, default_ms = None, None
     iters_done = 0
     if not args.no_tune:
-        # the stack under the default schedule (LDS tiles of 60 samples, 8
-        # backprojection rows): one iteration to build the plan, then as many
-        # timed as the tuned run below
+        # the stack under the default schedule of its single slices (LDS tiles of 60
+        # samples, 8 backprojection rows; slices in quads run the same under any): one
+        # iteration to build the plan, then as many timed as the tuned run below
         ctx.osem_batched(imgs, sinos, 1, use_graph=True)
         ctx.synchronize()
         with no_gc():
@@ -588,12 +588,12 @@ def main():
             default_ms = (time.perf_counter() - t0) * 1e3 / args.steps
         iters_done += 1 + args.steps
         log(f"default schedule: {default_ms:.1f} ms per step")
-        # then every side's own schedule (each side of a batched stack runs its own)
+        # then every side's own schedule (for its slices that are not in quads)
         tune = {m: ctx.autotune(m) for m in sorted(set(sides))}
         for m, t in tune.items():
             log(f"autotune side {m}: rays {t['fp_rays']} waves {t['fp_waves']} tile {t['fp_tile']} rows "
                 f"{t['bp_rows']}; FP {t['fp_ms']:.3f} ms (default {t['fp_ms_default']:.3f}), BP {t['bp_ms']:.3f} ms "
-                f"(default {t['bp_ms_default']:.3f}) on a batch-sized launch")
+                f"(default {t['bp_ms_default']:.3f}) on a batch-sized launch of single slices")
 
     # first call with the tuned schedules: one iteration
     ctx.osem_batched(imgs, sinos, 1, use_graph=True)
@@ -672,7 +672,6 @@ def main():
     kinds = sorted({(tune[m]["fp_rays"], tune[m]["fp_tile"]) for m in set(sides)} if tune else {(0, 60)})
     fp_kernel = " + ".join(f"k_fp_quad<FP_RATIO> (slices not in quads: k_fp_lds<FP_RATIO, {tile}>)" if rays == 0
                            else "k_fp<FP_RATIO>" for rays, tile in kinds)
-    fp_tile60 = kinds == [(0, 60)]
     fp_flops = sum(14.0 * m * na * m for m in sides)          # 14 FLOP per bilinear sample, D = m samples per ray
     fp_bytes = sum(4 * m * m + 8 * na * m for m in sides)    # image once, measured rows in, ratio rows out
     fp_tflops = fp_flops / (fp_ms * 1e-3) / 1e12
@@ -683,7 +682,7 @@ def main():
     roofline = {
         "bound": "valu", "achieved": round(fp_tflops, 3), "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
         "frac": round(fp_tflops / PEAK_FP32_TFLOPS, 4),
-        "traffic": (round(FP_TRAFFIC_BYTES_PER_SLICE * B) if uniform_1024 and fp_tile60 else None),
+        "traffic": (round(FP_TRAFFIC_BYTES_PER_SLICE * B) if uniform_1024 and B >= 4 else None),
         "algorithmic_bytes": fp_bytes,
         "kernel": f"{fp_kernel} (OSEM1: forward projection + ratio), timed per subset of every slice",
         "fp_ms_per_subset": round(fp_ms, 4), "bp_ms_per_subset": round(bp_ms, 4),
@@ -718,7 +717,7 @@ def main():
         "per_slice_launch": {"value": round(per_slice, 3), "unit": unit, "slices_timed": len(sample)},
         "batched_over_per_slice": round(value / per_slice, 3),
         "schedule_gain": (None if default_ms is None else
-                          {"default_ms_per_step": round(default_ms, 3),
+                          {"applies_to": "slices not in quads", "default_ms_per_step": round(default_ms, 3),
                            "tuned_ms_per_step": round(dt / args.steps * 1e3, 3),
                            "speedup": round(default_ms / (dt / args.steps * 1e3), 4)}),
         "roofline": roofline,

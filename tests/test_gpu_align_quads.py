@@ -16,9 +16,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("nx,ny,px,pa,dn,spread", [
     (64, 64, 64, 1800, 4, 1.5),                 # one chunk, one quad
     (97, 61, 130, 601, 6, 12.0),                # odd angles, one column over, a quad with two
-    (130, 171, 65, 903, 9, 0.0),                # one ray over, a layer left over
+    (130, 171, 65, 903, 9, 0.0),                # one ray over, a quad with one
     (301, 301, 256, 151, 11, 90.0),             # a quad with three, angles far apart in offset
-    (20, 33, 400, 257, 4, 5.0),                 # a detector much wider than the image
+    (20, 33, 400, 257, 4, 5.0),                 # a detector much wider than the image: single layers
 ])
 @pytest.mark.parametrize("deriv", [False, True])
 def test_quads_equal_single_layers(ctx, nx, ny, px, pa, dn, spread, deriv):

@@ -15,8 +15,9 @@ pytestmark = pytest.mark.gpu
 
 CASES = [
     # nx, ny, px, pa, ss, dn: at least 560 filled projection and 112 backprojection blocks run as quads
+    # (AART of so few subsets and blocks singly)
     (66, 53, 130, 130, 2, 58),                  # whole quads and one with two
-    (64, 64, 64, 180, 2, 113),                  # whole tiles; one slice left over
+    (64, 64, 64, 180, 2, 113),                  # whole tiles; a quad with one
     (127, 35, 65, 182, 2, 79),                  # one column short, three rows over, a quad with three
     (33, 130, 97, 90, 3, 5),                    # single slices only
     (65, 17, 40, 60, 4, 1),                     # one slice: it is its own layer neighbour

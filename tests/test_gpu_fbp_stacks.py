@@ -1,5 +1,5 @@
-"""FBP over the shapes its backprojection chooses kernels by: one row per block,
-8 and 16 rows per block, and interleaved quads of layers (whole, and with one
+"""FBP over shapes its backprojection chooses kernels by: 4 rows split over waves,
+16 rows per block, and interleaved quads of layers (whole, and with one
 or two empty places), on zero-padding lengths that are powers of 4 and twice
 them, odd grids and detectors narrower and wider than the grid.  Every layer
 against the oracle's FP32 restatement, to the 1e-5 of the single operators."""
@@ -15,8 +15,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,px,pa,zp,dn", [
     (2, 2, 3, 2, 1), (3, 3, 5, 4, 2), (8, 8, 5, 8, 1), (20, 17, 7, 32, 5),
     (129, 100, 23, 128, 3),       # 4 split rows per block, an odd angle count
-    (300, 390, 41, 512, 3),       # 8 rows per block
-    (257, 257, 24, 1024, 20),     # quads of 4 rows per block
+    (300, 390, 41, 512, 3),       # the same, a wide detector
+    (257, 257, 24, 1024, 20),     # whole quads of 16 rows per block, a pixel over
     (300, 260, 40, 512, 35),      # quads of 16 rows per block, the last with three layers
     (300, 260, 39, 512, 34),      # ... with two
     (300, 300, 25, 512, 33),      # ... and one layer singly

@@ -29,9 +29,9 @@ def _angles(kind, pa, rng):
     (129, 129, 129, 130, 2, 60, "full"),        # one ray, one pixel over
     (127, 127, 127, 240, 2, 35, "random"),      # a quad with three slices
     (150, 97, 170, 105, 1, 34, "wide"),         # rectangular, wide detector, a quad with two
-    (97, 150, 61, 300, 1, 33, "dense"),         # narrow detector, one slice left over
+    (97, 150, 61, 300, 1, 33, "dense"),         # narrow detector, a quad with one
     (20, 20, 20, 64, 1, 226, "random"),         # smaller than a chunk and a block
-    (512, 512, 512, 90, 1, 12, "wide"),
+    (512, 512, 512, 90, 1, 12, "wide"),         # angles too far apart for a window: single slices
     (1024, 1024, 1024, 240, 2, 4, "dense"),
 ])
 def test_quads_equal_single_slices(ctx, nx, ny, px, pa, ss, dn, kind):
