@@ -2513,7 +2513,7 @@ extern "C" ctr_status ctr_align_adjoint(ctr_ctx *c, const float *prj, const floa
     const ctr_geometry &g = c->g;
     HIPTRY(c, c->w_gpad.ensure(sizeof(float) * align_adj_floats(dN, g.nx, g.ny, g.pa, g.px)));
     launch_align_adjoint(prj, c->w_gpad.f(), static_cast<const float2 *>(c->cs.p), shifts, center, img, dN, g.nx,
-                         g.ny, g.pa, g.px, c->stream);
+                         g.ny, g.pa, g.px, c->cus, c->stream);
     POST(c, "align adjoint");
     return CTR_OK;
 }

@@ -176,7 +176,7 @@ void launch_align_quad(const float *img, const float *imgT, size_t ifl, size_t t
 constexpr int AD_PAD = 2;
 size_t align_adj_floats(int nz, int nx, int ny, int pa, int px);
 void launch_align_adjoint(const float *prj, float *gpad, const float2 *cs, const float *shifts, float center,
-                          float *img, int nz, int nx, int ny, int pa, int px, hipStream_t stream);
+                          float *img, int nz, int nx, int ny, int pa, int px, int cus, hipStream_t stream);
 void launch_align_grad(const float *pimg, const float *pimgT, int ipitch, int tpitch, const float2 *cs,
                        const float *gprj, const float *shifts, float center, float *partial, float *gshift,
                        int nz, int nx, int ny, int pa, int px, hipStream_t stream);
