@@ -804,10 +804,15 @@ constexpr long long QUAD_MIN_BP_BLOCKS = 112;
 constexpr int QUAD_INIT_PASSES = 8;
 constexpr long long QUAD_MIN_BP_BLOCKS_INIT = 320;
 // The two angles of a quad's projection block share a window while the rims of
-// their strips lie close: 21 x 1221^2, 23 angles (83 texels) take 1.25 times the
-// single slices' time, 4 x 2048^2, 40 angles (80) 0.96, 4 x 1536^2, 60 angles (40)
-// 0.86, 4 x 1024^2, 80 angles (20) 0.80.
-constexpr double QUAD_MAX_RIM_TEXELS = 56.0;
+// their strips lie close.  Single slices against quads, the ratio of their times: 4 x
+// 2048^2, 60 angles (54 texels) 1.31, 16 x 1221^2, 34 (56) 1.24, 12 x 1024^2, 28 (57) 1.08,
+// 4 x 2048^2, 50 (64) 1.22, 16 x 1024^2, 24 (67) 1.12, 48 x 512^2, 12 (67) 1.04, 24 x
+// 1024^2, 20 (80) 0.93, 8 x 1536^2, 30 (80) 1.14, 21 x 1221^2, 23 (83) 0.84, 8 x 2048^2, 30
+// (107) 0.96.  The alignment forward's blocks run in no such order and lose sooner,
+// without / with the derivative: 8 x 1484^2, 60 (39) 1.00 / 1.07, 4 x 2048^2, 80 (40) 1.02
+// / 1.12, 16 x 1024^2, 32 (50) 1.03 / 0.98, 12 x 1484^2 with 1024 bins, 45 (52) 0.95 / 0.99,
+// 4 x 2048^2, 60 (54) 0.92 / 0.88, 8 x 2048^2, 50 (64) 0.90 / 0.94.
+constexpr double QUAD_MAX_RIM_TEXELS = 70.0, ALIGN_MAX_RIM_TEXELS = 45.0;
 
 // blocks: projection blocks times the slices their quads hold, summed
 bool quads_fill(long long blocks, long long least) { return blocks >= QZ * least; }
@@ -2468,7 +2473,7 @@ ctr_status align_forward(ctr_ctx *c, const float *img, const float *shifts, floa
     std::vector<SliceSet *> sets;
     const int D = std::max(g.nx, g.ny);
     int nq = align_quads_of(dN, g.nx, g.ny, g.px, g.pa);
-    if (nq > 0 && !(rim_texels(c, D, 1) <= QUAD_MAX_RIM_TEXELS)) nq = 0;
+    if (nq > 0 && !(rim_texels(c, D, 1) <= ALIGN_MAX_RIM_TEXELS)) nq = 0;
     TRY(split_stack(c, dN, nq, false, b, sets));
     for (SliceSet *S : sets) {
         TRY(run_kind(c, *S, G_PAD));

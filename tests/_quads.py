@@ -1,13 +1,17 @@
 """The library's choice between quads (four slices side by side) and single slices:
 its own functions, called on the host, and the distance of the angles restated."""
 import ctypes
+import os
+import re
 
 import numpy as np
 import torch  # noqa: F401  (its HIP runtime is the one to load first)
-from ctrecon import load
+from ctrecon import _lib, load
 
 _LIB = load()
-MAX_RIM_TEXELS = 56.0
+with open(os.path.join(os.path.dirname(_lib.__file__), "..", "csrc", "ctr_api.cpp")) as _f:
+    MAX_RIM_TEXELS, ALIGN_MAX_RIM_TEXELS = (float(v) for v in re.search(
+        r"QUAD_MAX_RIM_TEXELS = ([0-9.]+), ALIGN_MAX_RIM_TEXELS = ([0-9.]+);", _f.read()).groups())
 
 
 def rim_texels(ang, D, stride):
@@ -27,7 +31,7 @@ def stack_quads(nx, ny, px, pa, ss, dn, ang, passes=2 ** 31 - 1):
 def align_quads(nx, ny, px, pa, dn, ang):
     """Layers of an alignment forward that run as quads."""
     nq = _LIB._ZN3ctr14align_quads_ofEiiiii(dn, nx, ny, px, pa)
-    return nq if nq and rim_texels(ang, max(nx, ny), 1) <= MAX_RIM_TEXELS else 0
+    return nq if nq and rim_texels(ang, max(nx, ny), 1) <= ALIGN_MAX_RIM_TEXELS else 0
 
 
 def fbp_kernels(nx, ny, zp, dn):

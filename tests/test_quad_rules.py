@@ -32,3 +32,12 @@ def test_batches():
     assert _quads.batch_quads([445] * 8 + [524] * 12 + [713] * 4, 30) == 24       # 795
     assert _quads.batch_quads([1024] * 17, 45) == 16
     assert _quads.batch_quads([512] * 8, 80) == 8
+
+
+def test_angles_far_apart():
+    def turn(pa):
+        return np.arange(pa) * (180.0 / pa)
+    assert _quads.stack_quads(2048, 2048, 2048, 50, 1, 4, turn(50)) == 4        # rims 64 texels apart
+    assert _quads.stack_quads(1024, 1024, 1024, 20, 1, 24, turn(20)) == 0       # 80
+    assert _quads.align_quads(2048, 2048, 2048, 80, 4, turn(80)) == 4           # 40
+    assert _quads.align_quads(2048, 2048, 2048, 60, 4, turn(60)) == 0           # 54
