@@ -331,7 +331,8 @@ ctr_status ctr_tv_prox_2d(ctr_ctx *ctx, const float *v, float *x_new, int dN, fl
 
 /* Runs OS-EM (OSEM_execution semantics, no correction) on `count` slices of
  * possibly different sides in one stream-ordered schedule: per subset, one
- * launch per kernel covers every slice.  use_graph != 0 captures one
+ * launch per kernel covers every slice that runs four side by side, and one
+ * per distinct schedule the others.  use_graph != 0 captures one
  * iteration in a hipGraph and replays it.  Workspace and graphs are cached
  * in the context for repeated calls with the same slice list. */
 ctr_status ctr_osem_batched(ctr_ctx *ctx, const ctr_slice *slices, int count, int it,
@@ -340,7 +341,8 @@ ctr_status ctr_osem_batched(ctr_ctx *ctx, const ctr_slice *slices, int count, in
 /* A projector / backprojector schedule for one slice side.  It applies to
  * slices that run one by one; where a side has enough of them, OS-EM, TV OS-EM,
  * AART and batched stacks run four slices side by side with a shape of their
- * own (the same images bit for bit as under the LDS-tiled schedules).  No
+ * own (the same images bit for bit as under the LDS-tiled schedules; direct
+ * gathers sum a ray in another order and differ in the last bits).  No
  * reference counterpart: the reference fixes its work-group shape per compiled
  * program (GPU.cpp:169-172, 538-547). */
 typedef struct ctr_schedule {
@@ -376,7 +378,9 @@ ctr_status ctr_get_schedule(ctr_ctx *ctx, int n, ctr_schedule *schedule);
 ctr_status ctr_set_adaptive_rows(ctr_ctx *ctx, int enable);
 
 /* Average duration (ms) of the last timed forward-projection and
- * backprojection launches recorded with ctr_set_kernel_timing(ctx, 1). */
+ * backprojection launches recorded with ctr_set_kernel_timing(ctx, 1).  A stack
+ * that runs partly four slices side by side and partly singly is two launches
+ * of each kind per subset. */
 ctr_status ctr_set_kernel_timing(ctr_ctx *ctx, int enable);
 ctr_status ctr_kernel_timing(ctr_ctx *ctx, double *fp_ms, double *bp_ms, int *fp_launches,
                              int *bp_launches);
